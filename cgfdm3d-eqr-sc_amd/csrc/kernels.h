@@ -21,8 +21,9 @@ struct StageArgs {
   const float* aff;     // 16-bit coefficient storage: affine table [12][NZ][2] (mid, half); else unused
   int nzp;              // padded z extent (rows of the affine table)
   const R* win;         // stencil input (9 SoA fields)
-  const R* wm;          // RK base (state at the start of the step)
-  R* wt;                // RK accumulator
+  const R* wm;          // RK base (state at the start of the step; the last stage's output)
+  const R* x1;          // states of stages 1 and 2, read by the last stage
+  const R* x2;
   R* wout;              // stage output
   PmlArgs<R> pml;
 };

@@ -92,7 +92,7 @@ int launch_interior(StageArgs<R> a, const TM* coef, int fb1, int fb2, int fb3, h
   if constexpr (std::is_same<R, float>::value && std::is_same<TM, float>::value) {
     // 8-byte pair accesses need every array's even columns on 8-byte boundaries
     auto al8 = [](const void* q) { return (reinterpret_cast<unsigned long long>(q) & 7) == 0; };
-    if (a.kc < 0 && a.NX % 2 == 0 && a.N % 2 == 0 && al8(a.win) && al8(a.wout) && al8(a.wm) && al8(a.wt) && al8(coef)) {
+    if (a.kc < 0 && a.NX % 2 == 0 && a.N % 2 == 0 && al8(a.win) && al8(a.wout) && al8(a.wm) && al8(a.x1) && al8(a.x2) && al8(coef)) {
       // x-paired kernel: 128 x 4 cells per block, 8-byte accesses
       const long long nb = (long long)((a.nx + 1 + 127) / 128) * ((a.ny + 3) / 4) * nk;
       if (nb > 0x7fffffffLL) return LAUNCH_TOO_LARGE;
