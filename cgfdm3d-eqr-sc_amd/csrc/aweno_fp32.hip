@@ -1,5 +1,5 @@
 // FP32 instantiation of the ME-AWENO step kernels.
-#include "aweno_impl.h"
+#include "aweno_march.h"
 
 namespace aw {
 template void launch_faces<float>(const StageArgs<float>&, hipStream_t);

@@ -146,11 +146,11 @@ __device__ __forceinline__ R pl(const R* base, long long N, int c, unsigned o) {
   return *at(base + (long long)c * N, o);
 }
 
-// Lax-Friedrichs face flux of direction d at face q+1/2, stored at cell q
+// Lax-Friedrichs face flux of direction d at face q+1/2
 // (wave_deriv_alternative_flux_FD_{x,y,z}); o is the byte offset of cell q,
 // sb the byte stride of direction d.
 template <class R>
-__device__ __forceinline__ void face_flux(const StageArgs<R>& a, unsigned o, unsigned sb, int d) {
+__device__ __forceinline__ void face_values(const StageArgs<R>& a, unsigned o, unsigned sb, int d, R (&F)[9]) {
   const long long N = a.N;
   const R n1 = pl(a.cjm, N, 3 * d + 0, o), n2 = pl(a.cjm, N, 3 * d + 1, o), n3 = pl(a.cjm, N, 3 * d + 2, o);
   const R mu = pl(a.cjm, N, C_MU, o), lam = pl(a.cjm, N, C_LAM, o), b = pl(a.cjm, N, C_B, o);
@@ -167,25 +167,36 @@ __device__ __forceinline__ void face_flux(const StageArgs<R>& a, unsigned o, uns
       up[v] = weno5<R>(wp3, wp2, wp1, w0, wm1);
     }
   }
-  R* F = a.F + (long long)(9 * d) * N;
   if constexpr (sizeof(R) == 4) {
     // the flux is linear in the state: F(u+) + F(u-) = F(u+ + u-), one flux
     // evaluation per face instead of two (equal up to rounding)
-    R us[9], fs[9];
+    R us[9];
 #pragma unroll
     for (int v = 0; v < 9; ++v) us[v] = up[v] + um[v];
-    phys_flux<R>(us, n1, n2, n3, mu, lam, b, fs);
+    phys_flux<R>(us, n1, n2, n3, mu, lam, b, F);
 #pragma unroll
-    // non-temporal: the flux planes stream out and back in the update kernel
-    // without displacing the state rows the neighbouring faces re-read
-    for (int v = 0; v < 9; ++v)
-      __builtin_nontemporal_store(R(R(0.5) * (fs[v] - a.alpha * (up[v] - um[v]))), at(F + v * N, o));
+    for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (F[v] - a.alpha * (up[v] - um[v]));
   } else {
     R fm[9], fp[9];
     phys_flux<R>(um, n1, n2, n3, mu, lam, b, fm);
     phys_flux<R>(up, n1, n2, n3, mu, lam, b, fp);
 #pragma unroll
-    for (int v = 0; v < 9; ++v) *at(F + v * N, o) = R(0.5) * (fp[v] + fm[v] - a.alpha * (up[v] - um[v]));
+    for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (fp[v] + fm[v] - a.alpha * (up[v] - um[v]));
+  }
+}
+
+// the same, stored at cell q of the flux array
+template <class R>
+__device__ __forceinline__ void face_flux(const StageArgs<R>& a, unsigned o, unsigned sb, int d) {
+  R f[9];
+  face_values<R>(a, o, sb, d, f);
+  R* F = a.F + (long long)(9 * d) * a.N;
+  // FP32, non-temporal: the flux planes stream out and back in the update kernel
+  // without displacing the state rows the neighbouring faces re-read
+#pragma unroll
+  for (int v = 0; v < 9; ++v) {
+    if constexpr (sizeof(R) == 4) __builtin_nontemporal_store(f[v], at(F + v * a.N, o));
+    else *at(F + v * a.N, o) = f[v];
   }
 }
 
@@ -322,8 +333,12 @@ __global__ void __launch_bounds__(256) aw_update(StageArgs<R> a) {
 
 // The three interior layers under the top: the corrections use 6-point
 // formulas on the physical fluxes of the 7 cells around the cell
-// (alternative_flux_FD.cpp:1257-1278), in every direction.
-template <class R>
+// (alternative_flux_FD.cpp:1257-1278), in every direction. OWNF: there is no
+// flux array, a cell evaluates its six face fluxes itself (twice the work, on
+// three layers, beside the marching kernels), and the z blocks 3..5 carry the
+// ghost cells above the interior through the stage, which the free surface
+// rewrites every step (no right-hand side; the other ghost cells never change).
+template <class R, bool OWNF>
 __global__ void __launch_bounds__(256) aw_update_top(StageArgs<R> a, int nx, int ny) {
   const int i = H + blockIdx.x * 64 + (threadIdx.x & 63);
   const int j = H + blockIdx.y * 4 + (threadIdx.x >> 6);
@@ -331,6 +346,19 @@ __global__ void __launch_bounds__(256) aw_update_top(StageArgs<R> a, int nx, int
   if (i >= H + nx || j >= H + ny) return;
   const long long N = a.N;
   const long long p = (long long)i + (long long)a.NX * j + (long long)k * a.S;
+  if constexpr (OWNF) {
+    if (k >= a.NZ - H) {
+      R mv[9], wv[9];
+#pragma unroll
+      for (int v = 0; v < 9; ++v) {
+        mv[v] = a.wm[v * N + p];
+        wv[v] = a.win[v * N + p];
+      }
+#pragma unroll
+      for (int v = 0; v < 9; ++v) a.wout[v * N + p] = tvd<R>(a.stage, mv[v], wv[v], R(0));
+      return;
+    }
+  }
   const R jac = R(1.0 / (double)a.cjm[C_J * N + p]);
   const R cd = a.DT * a.rDH * jac;
   R h[9];
@@ -348,12 +376,24 @@ __global__ void __launch_bounds__(256) aw_update_top(StageArgs<R> a, int nx, int
       phys_flux<R>(u, a.cjm[(3 * d) * N + q], a.cjm[(3 * d + 1) * N + q], a.cjm[(3 * d + 2) * N + q],
                    a.cjm[C_MU * N + q], a.cjm[C_LAM * N + q], a.cjm[C_B * N + q], hu[n]);
     }
-    const R* F = a.F + (long long)(9 * d) * N;
+    R F0[9], F1[9];  // faces after and before the cell
+    if constexpr (OWNF) {
+      const unsigned sb = d == 0 ? (unsigned)sizeof(R) : d == 1 ? a.rowb : a.planeb, o = (unsigned)(p * (long long)sizeof(R));
+      face_values<R>(a, o, sb, d, F0);
+      face_values<R>(a, o - sb, sb, d, F1);
+    } else {
+      const R* F = a.F + (long long)(9 * d) * N;
+#pragma unroll
+      for (int v = 0; v < 9; ++v) {
+        F0[v] = F[v * N + p];
+        F1[v] = F[v * N + p - s];
+      }
+    }
 #pragma unroll
     for (int v = 0; v < 9; ++v) {
-      const R fr = F[v * N + p] - R(1.0 / 24.0) * d2f<R>(hu[1][v], hu[2][v], hu[3][v], hu[4][v], hu[5][v], hu[6][v]) +
+      const R fr = F0[v] - R(1.0 / 24.0) * d2f<R>(hu[1][v], hu[2][v], hu[3][v], hu[4][v], hu[5][v], hu[6][v]) +
                    R(7.0 / 5760.0) * d4f<R>(hu[1][v], hu[2][v], hu[3][v], hu[4][v], hu[5][v], hu[6][v]);
-      const R fl = F[v * N + p - s] - R(1.0 / 24.0) * d2f<R>(hu[0][v], hu[1][v], hu[2][v], hu[3][v], hu[4][v], hu[5][v]) +
+      const R fl = F1[v] - R(1.0 / 24.0) * d2f<R>(hu[0][v], hu[1][v], hu[2][v], hu[3][v], hu[4][v], hu[5][v]) +
                    R(7.0 / 5760.0) * d4f<R>(hu[0][v], hu[1][v], hu[2][v], hu[3][v], hu[4][v], hu[5][v]);
       h[v] += cd * (-(fr - fl));
     }
@@ -632,7 +672,7 @@ void launch_update(const StageArgs<R>& a, int nx, int ny, hipStream_t st, hipStr
   // write disjoint cells and read only the stage input and the face fluxes
   const dim3 block(256);
   const dim3 gtop((nx + 63) / 64, (ny + 3) / 4, 3);
-  aw_update_top<R><<<gtop, block, 0, st_top>>>(a, nx, ny);
+  aw_update_top<R, false><<<gtop, block, 0, st_top>>>(a, nx, ny);
   const long long nb = cg::interior_blocks(a.XE - 2 * H, a.NY, a.NZ, a.rtx, a.rty);
   aw_update<R><<<dim3((unsigned)nb), block, 0, st>>>(a);
 }

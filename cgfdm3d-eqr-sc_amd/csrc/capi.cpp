@@ -1353,6 +1353,11 @@ struct AwenoSolver : SolverBase {
   // CGFDM_INTERIOR_RTX (0..64) / _RTY (1..64) override it
   int rty = 2;
   int rtx = 0;
+  // FP32: marching kernels without the flux array (aweno_march.h) from 400000
+  // cells on, where they have enough columns to fill the chip: us per stage
+  // 97 against 66 at 64 x 60 x 40, 131 against 156 at 96 x 90 x 60, 1395 against
+  // 2070 at 512 x 500 x 60. CGFDM_AWENO_MARCH (0 or 1) overrides the rule.
+  bool march = false;
 
   int init(const cgfdm_desc& dd, const float* coord, const float* medium) override {
     d = dd;
@@ -1415,7 +1420,9 @@ struct AwenoSolver : SolverBase {
     dfree(cjm_t);
     for (int q = 0; q < 3; ++q)
       if ((rc = galloc(&buf[q], 9 * N))) return rc;
-    if ((rc = galloc(&F, 27 * N))) return rc;
+    march = sizeof(R) == 4 && (double)d.nx * d.ny * d.nz >= 400000.0;
+    if (const char* e = std::getenv("CGFDM_AWENO_MARCH")) march = sizeof(R) == 4 && std::atoi(e) != 0;
+    if (!march && (rc = galloc(&F, 27 * N))) return rc;
     if ((rc = dalloc(&pgv, 2LL * d.nx * d.ny))) return rc;
     if ((rc = dalloc(&dis, 3 * S))) return rc;
     HIPCHK(hipStreamSynchronize(stream));
@@ -1485,11 +1492,11 @@ struct AwenoSolver : SolverBase {
   }
 
   const char* kernel_name(int which) const override {
-    return which == 0 ? "aw_faces" : which == 1 ? "aw_update" : nullptr;
+    return which == 0 ? (march ? "aw_yflux" : "aw_faces") : which == 1 ? (march ? "aw_xzstep" : "aw_update") : nullptr;
   }
 
   int step(int n) override {
-    if (surf_overlap && !sstream) {
+    if (surf_overlap && !march && !sstream) {
       HIPCHK(hipStreamCreateWithFlags(&sstream, hipStreamNonBlocking));
       HIPCHK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
       HIPCHK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
@@ -1540,11 +1547,20 @@ struct AwenoSolver : SolverBase {
           fp = next_pair(0);
           HIPCHK(hipEventRecord(ev[fp].a, stream));
         }
-        aw::launch_faces<R>(a, stream);
+        if (march) {
+          if constexpr (sizeof(R) == 4) aw::launch_march_y(a, d.nx, d.ny, stream);
+        } else {
+          aw::launch_faces<R>(a, stream);
+        }
         if (timing_on) {
           HIPCHK(hipEventRecord(ev[fp].b, stream));
           up = next_pair(1);
           HIPCHK(hipEventRecord(ev[up].a, stream));
+        }
+        if (march) {
+          if constexpr (sizeof(R) == 4) aw::launch_march_xz(a, d.nx, d.ny, stream);
+          if (timing_on) HIPCHK(hipEventRecord(ev[up].b, stream));
+          continue;
         }
         if (surf_overlap) {
           HIPCHK(hipEventRecord(ev_fork, stream));
@@ -1643,7 +1659,13 @@ struct AwenoSolver : SolverBase {
     HIPCHK(hipStreamSynchronize(stream));
     std::vector<R> h(tN);
     for (long long p = 0; p < tN; ++p) h[p] = R(in[p]);
-    return to_dev(buf[cur] + (size_t)comp * N, h.data(), 1);
+    if (int rc = to_dev(buf[cur] + (size_t)comp * N, h.data(), 1)) return rc;
+    // the marching stages leave the ghost cells of their output buffers alone
+    if (march)
+      for (int q = 1; q < 3; ++q)
+        HIPCHK(hipMemcpyAsync(buf[(cur + q) % 3] + (size_t)comp * N, buf[cur] + (size_t)comp * N, sizeof(R) * N,
+                              hipMemcpyDeviceToDevice, stream));
+    return CGFDM_OK;
   }
 
   int get_setup(int what, double* out) override {

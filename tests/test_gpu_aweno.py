@@ -89,3 +89,31 @@ def test_aweno_fp32_seismograms_vs_fp64_oracle(oracle_mod, solver_mod):
     sg, so = g.stations(), o.stations()
     assert rel_l2(sg[..., :3], so[..., :3]) < 1e-4
     assert rel_l2(g.pgv(), o.pgv()) < 1e-4
+
+
+# Marching kernels against the kernels with the flux array: one wave of columns
+# exactly (nx 58) and one more (59), full and partial second and third waves, the
+# shallowest grids (one to three planes below the top layers), several chunks
+# along y and z. Both sides evaluate the same FP32 scheme in another order; the
+# tolerance is that of the FP32 comparison with the oracle.
+@pytest.mark.parametrize("nx,ny,nz,fs", [(58, 9, 4, True), (59, 12, 5, False), (6, 5, 6, True), (66, 40, 9, True),
+                                         (112, 7, 30, False), (113, 33, 14, True), (24, 90, 61, True)])
+def test_aweno_marching_kernels_match_the_flux_array(solver_mod, monkeypatch, nx, ny, nz, fs):
+    m = M.small_config(nx=nx, ny=ny, nz=nz, npml=0, hills=2, layered=True, free_surface=fs, nt=8)
+    m.stations = m.stations[:2]
+    rng = np.random.default_rng(nx * 1000 + ny)
+    shape = (nz + 2 * H, ny + 2 * H, nx + 2 * H)
+    # ghost cells carry values too: the stages hand them on
+    init = [rng.standard_normal(shape) * (100.0 if v < 3 else 1e-5) for v in range(9)]
+    out = []
+    for march in ("0", "1"):
+        monkeypatch.setenv("CGFDM_AWENO_MARCH", march)
+        print(f"march={march} {nx}x{ny}x{nz} fs={fs}", flush=True)
+        g = solver_mod.Solver(m, precision=4, scheme=solver_mod.SCHEME_AWENO)
+        assert g.kernel_name(0) == ("aw_yflux" if march == "1" else "aw_faces")
+        for v in range(9):
+            g.set_field(v, init[v])
+        g.step(4)
+        out.append(g.wavefield())
+    for v in range(9):
+        assert rel_l2(out[1][v], out[0][v]) < 1e-5, (v, rel_l2(out[1][v], out[0][v]))
