@@ -81,24 +81,34 @@ __device__ __forceinline__ R mac(const R* f, long long s) {
                   R(AF3) * f[3 * FB * s]);
 }
 
+// Keeps the compiler from moving loads issued before this point behind the
+// arithmetic that follows: to save registers it otherwise serialises a group of
+// loads (load, wait, use, up to 45 times over) in some instances of a kernel. The
+// first stage with F/B (+, +, .) took 4.3 ms at 512 x 512 x 256 for the bytes that
+// other signs moved in 3.0; with all groups fixed every first stage takes 2.8, and a
+// step in FP64 at 200 x 180 x 100 2.8 -> 2.6 ms.
+__device__ __forceinline__ void loads_issued() { __builtin_amdgcn_sched_barrier(0); }
+
 // CFS-PML auxiliary update for one face at slab index pos (reference
-// pml_deriv.cpp:235-273 and pml_rk.cpp:19-73): hA = (d Q - (alpha+d) A) DT,
+// pml_deriv.cpp:235-273 and pml_rk.cpp:19-73): hA = (d Q - (al+d) A) DT,
 // h -= beta A DT, then the RK4 stage on the auxiliary state. The stage is a
 // compile-time parameter: every kernel instance has one straight-line memory
 // pattern and no stage-dependent choice of base pointers.
 template <class R, int STAGE>
-__device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, const R (&Q)[9], R d, R ad, R be, R DT,
+__device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, const R (&Q)[9], R d, R al, R be, R DT,
                                          R (&h)[9], bool has_extra, const R (&extra)[6]) {
   // extra: surface stress term added to hA[3..8] on the top layer.
-  // The nine fields go in three groups of three, each group's loads before its
-  // stores: the buffers are not known not to alias, so a store between two
-  // loads would make the compiler wait for each load in turn (three round
-  // trips instead of nine, with few registers held).
+  // Loads before stores: the buffers are not known not to alias, so a store between
+  // two loads would make the compiler wait for each load in turn. All nine fields
+  // together (five and four in the last stage, which reads four buffers): the
+  // stencil's registers are free at this point.
+  constexpr int G = STAGE == 3 ? 5 : 9;
 #pragma unroll
-  for (int g = 0; g < 9; g += 3) {
-    R cur[3], av[3], x1[3], x2[3];
+  for (int g = 0; g < 9; g += G) {
+    R cur[G], av[G], x1[G], x2[G];
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
+    for (int u = 0; u < G; ++u) {
+      if (g + u >= 9) break;
       const long long q = (long long)(g + u) * F.cnt + pos;
       cur[u] = (STAGE == 0 ? F.a : STAGE == 1 ? F.x1 : STAGE == 2 ? F.x2 : F.x3)[q];
       if constexpr (STAGE != 0) av[u] = F.a[q];
@@ -107,9 +117,12 @@ __device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, con
         x2[u] = F.x2[q];
       }
     }
+    loads_issued();
+    const R ad = d + al;
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
+    for (int u = 0; u < G; ++u) {
       const int v = g + u;
+      if (v >= 9) break;
       const long long q = (long long)v * F.cnt + pos;
       R hA = (d * Q[v] - ad * cur[u]) * DT;
       if (has_extra && v >= 3) hA += extra[v - 3] * DT;
@@ -123,11 +136,12 @@ __device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, con
 }
 
 // ---------------------------------------------------------------------------
-// interior cell update: 27 derivatives, PML faces, RK4 stage. `xd(v)`, `yd(v)`
-// and `zd(v)` return the unscaled xi, eta and zeta differences of field v and
-// `wc(v)` the centre value, so the same body serves the thread-per-cell kernel
-// (differences from global memory) and the z-marching kernel (x/y from an LDS
-// plane, z from a register window).
+// interior cell update: 27 derivatives, PML faces, RK4 stage. `xt(v, f)`,
+// `yt(v, f)` and `zt(v, f)` fetch the stencil of field v along an axis: f[0] one
+// cell against the F/B direction, f[2..4] one to three cells along it, and xt also
+// f[1], the centre. The same body thus serves the thread-per-cell kernel (from
+// global memory) and the z-marching ones (from an LDS plane or registers). All of
+// an axis' loads are issued before its arithmetic.
 // ---------------------------------------------------------------------------
 // Streaming accesses of a stage (coefficients, RK base and accumulator, the
 // two outputs) are used once per cell: they carry the non-temporal hint so
@@ -145,34 +159,71 @@ __device__ __forceinline__ unsigned cell_off(const StageArgs<R>& a, int i, int j
   return (unsigned)i * (unsigned)sizeof(R) + (unsigned)j * a.rowb + (unsigned)k * a.planeb;
 }
 
-// 5-point MacCormack difference (without 1/DH) of one plane array around byte
-// offset o with a byte stride st between stencil points.
+// Stencil of one plane array around byte offset o with a byte stride st between
+// its points; the centre f[1] is left to the caller.
 template <int FB, class R>
-__device__ __forceinline__ R mac_off(const R* base, unsigned o, unsigned st) {
+__device__ __forceinline__ void taps_off(const R* base, unsigned o, unsigned st, R* f) {
   const unsigned d = FB > 0 ? st : 0u - st;
-  return R(FB) * (R(AF_1) * *at(base, o - d) + R(AF0) * *at(base, o) + R(AF1) * *at(base, o + d) +
-                  R(AF2) * *at(base, o + 2 * d) + R(AF3) * *at(base, o + 3 * d));
+  f[0] = *at(base, o - d);
+  f[2] = *at(base, o + d);
+  f[3] = *at(base, o + 2 * d);
+  f[4] = *at(base, o + 3 * d);
+}
+// the same from a pointer to the centre and an element stride
+template <int FB, class R>
+__device__ __forceinline__ void taps(const R* c, long long s, R* f) {
+  f[0] = c[-FB * s];
+  f[2] = c[FB * s];
+  f[3] = c[2 * FB * s];
+  f[4] = c[3 * FB * s];
 }
 
-// Coefficient c of the cell at byte offset `off` in layer k. Native storage:
-// plane c (with the non-temporal hint when NT is set). 16-bit storage: the half
-// of word plane c / 2 that holds plane c, decoded with the layer's affine pair.
-template <class R, class TM, bool NT>
-__device__ __forceinline__ R coef_off(const TM* __restrict__ coef, const StageArgs<R>& a, int c, unsigned off, int k) {
-  if constexpr (sizeof(TM) == 2) {
-    static_assert(sizeof(R) == 4, "16-bit coefficient words are addressed like an FP32 grid array");
-    const unsigned* w = at(reinterpret_cast<const unsigned*>(coef) + (long long)(c >> 1) * a.N, off);
-    const unsigned word = NT ? __builtin_nontemporal_load(w) : *w;
-    const unsigned short b = (c & 1) ? (unsigned short)(word >> 16) : (unsigned short)(word & 0xffffu);
-    const float* A = a.aff + 2 * ((long long)c * a.nzp + k);
-    return R(A[0] + A[1] * Bits16<TM>::to_float(b));
-  } else {
-    static_assert(sizeof(TM) == sizeof(R), "native coefficients share the grid byte offsets");
-    const TM* q = at(coef + (long long)c * a.N, off);
-    if constexpr (NT) return R(__builtin_nontemporal_load(q));
-    else return R(*q);
+// Coefficients of the cell at byte offset `off` in layer k, loaded axis by axis
+// (axis 0 with mu, lambda and 1/rho). Native storage: plane c, non-temporal.
+template <class R, class TM>
+struct CellCoef {
+  static_assert(sizeof(TM) == sizeof(R), "native coefficients share the grid byte offsets");
+  TM r[M_NCOEF];
+  __device__ __forceinline__ void load1(const TM* __restrict__ coef, long long N, unsigned off, int c) {
+    r[c] = __builtin_nontemporal_load(at(coef + (long long)c * N, off));
   }
-}
+  __device__ __forceinline__ void load(const TM* __restrict__ coef, const StageArgs<R>& a, unsigned off, int axis) {
+#pragma unroll
+    for (int c = 3 * axis; c < 3 * axis + 3; ++c) load1(coef, a.N, off, c);
+    if (axis == 0)
+#pragma unroll
+      for (int c = M_MU; c <= M_B; ++c) load1(coef, a.N, off, c);
+  }
+  __device__ __forceinline__ R get(const StageArgs<R>&, int c, int) const { return R(r[c]); }
+};
+// 16-bit storage: the half of word plane c / 2 that holds plane c, decoded with
+// the layer's affine pair. Word 1 holds xi_z and eta_x, word 4 zeta_z and mu.
+template <class TM>
+struct CellCoef16 {
+  unsigned w[M_NCOEF / 2];
+  __device__ __forceinline__ void load1(const TM* __restrict__ coef, long long N, unsigned off, int q) {
+    w[q] = __builtin_nontemporal_load(at(reinterpret_cast<const unsigned*>(coef) + (long long)q * N, off));
+  }
+  __device__ __forceinline__ void load(const TM* __restrict__ coef, const StageArgs<float>& a, unsigned off, int axis) {
+    if (axis == 0) {
+      load1(coef, a.N, off, 0);
+      load1(coef, a.N, off, 1);
+      load1(coef, a.N, off, 4);
+      load1(coef, a.N, off, 5);
+    } else {
+      load1(coef, a.N, off, axis + 1);
+    }
+  }
+  __device__ __forceinline__ float get(const StageArgs<float>& a, int c, int k) const {
+    const unsigned short b = (c & 1) ? (unsigned short)(w[c >> 1] >> 16) : (unsigned short)(w[c >> 1] & 0xffffu);
+    const float* A = a.aff + 2 * ((long long)c * a.nzp + k);
+    return A[0] + A[1] * Bits16<TM>::to_float(b);
+  }
+};
+template <>
+struct CellCoef<float, __half> : CellCoef16<__half> {};
+template <>
+struct CellCoef<float, __hip_bfloat16> : CellCoef16<__hip_bfloat16> {};
 
 // Coefficient c of cell q (linear index, in layer k), for the surface kernel.
 template <class R, class TM, bool NT>
@@ -190,20 +241,35 @@ __device__ __forceinline__ R coef_at(const TM* __restrict__ coef, const StageArg
   }
 }
 
-template <class R, class TM, int FB1, int FB2, int FB3, int STAGE, class XD, class YD, class ZD, class WC>
+template <class R, class TM, int FB1, int FB2, int FB3, int STAGE, class XT, class YT, class ZT>
 __device__ __forceinline__ void cell_body(const StageArgs<R>& a, const TM* __restrict__ coef, int i, int j, int k,
-                                          unsigned off, XD xd, YD yd, ZD zd, WC wc) {
+                                          unsigned off, XT xt, YT yt, ZT zt) {
   const long long N = a.N;
-  auto cf = [&](int c) -> R { return coef_off<R, TM, true>(coef, a, c, off, k); };
-  const R mu = cf(M_MU), lam = cf(M_LAM), bu = cf(M_B);
+  CellCoef<R, TM> cc;
+  auto cf = [&](int c) -> R { return cc.get(a, c, k); };
   const PmlArgs<R>& P = a.pml;
-  R h[9], D[9], Q[9];
+  R h[9], D[9], Q[9], ctr[9], bx, by, bz;
+  // differences of all fields from the fetched stencils
+  auto diff = [&](int fb, const R (&f)[9][5]) {
+#pragma unroll
+    for (int v = 0; v < 9; ++v)
+      D[v] = R(fb) * (R(AF_1) * f[v][0] + R(AF0) * ctr[v] + R(AF1) * f[v][2] + R(AF2) * f[v][3] + R(AF3) * f[v][4]);
+  };
 
   // x: derivatives along xi (wave_deriv.cpp:214-222), scaled by 1/beta_x
+  {
+    R f[9][5];
 #pragma unroll
-  for (int v = 0; v < 9; ++v) D[v] = xd(v);
+    for (int v = 0; v < 9; ++v) xt(v, f[v]);
+    cc.load(coef, a, off, 0);
+    bx = P.beta[0][i];
+    loads_issued();
+#pragma unroll
+    for (int v = 0; v < 9; ++v) ctr[v] = f[v][1];
+    diff(FB1, f);
+  }
+  const R mu = cf(M_MU), lam = cf(M_LAM), bu = cf(M_B);
   assemble(D, cf(M_XIX), cf(M_XIY), cf(M_XIZ), mu, lam, bu, Q);
-  const R bx = P.beta[0][i];
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
     Q[v] *= a.rDH;
@@ -213,17 +279,23 @@ __device__ __forceinline__ void cell_body(const StageArgs<R>& a, const TM* __res
   if (P.npml > 0) {
     const bool x1 = i < H + P.npml, x2 = i >= H + a.nx - P.npml;
     if (x1 || x2) {
-      const R d = P.d[0][i], ad = d + P.alpha[0][i];
+      const R d = P.d[0][i], al = P.alpha[0][i];
       const long long row = (long long)(j - H) + (long long)a.ny * (k - H);
-      if (x1) pml_face<R, STAGE>(P.f[0], (long long)(i - H) + (long long)P.npml * row, Q, d, ad, bx, a.DT, h, false, none);
-      if (x2) pml_face<R, STAGE>(P.f[3], (long long)(i - H - (a.nx - P.npml)) + (long long)P.npml * row, Q, d, ad, bx, a.DT, h, false, none);
+      if (x1) pml_face<R, STAGE>(P.f[0], (long long)(i - H) + (long long)P.npml * row, Q, d, al, bx, a.DT, h, false, none);
+      if (x2) pml_face<R, STAGE>(P.f[3], (long long)(i - H - (a.nx - P.npml)) + (long long)P.npml * row, Q, d, al, bx, a.DT, h, false, none);
     }
   }
   // y: derivatives along eta (wave_deriv.cpp:224-232)
+  {
+    R f[9][5];
 #pragma unroll
-  for (int v = 0; v < 9; ++v) D[v] = yd(v);
+    for (int v = 0; v < 9; ++v) yt(v, f[v]);
+    cc.load(coef, a, off, 1);
+    by = P.beta[1][j];
+    loads_issued();
+    diff(FB2, f);
+  }
   assemble(D, cf(M_ETX), cf(M_ETY), cf(M_ETZ), mu, lam, bu, Q);
-  const R by = P.beta[1][j];
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
     Q[v] *= a.rDH;
@@ -232,17 +304,23 @@ __device__ __forceinline__ void cell_body(const StageArgs<R>& a, const TM* __res
   if (P.npml > 0) {
     const bool y1 = j < H + P.npml, y2 = j >= H + a.ny - P.npml;
     if (y1 || y2) {
-      const R d = P.d[1][j], ad = d + P.alpha[1][j];
+      const R d = P.d[1][j], al = P.alpha[1][j];
       const long long i0 = i - H, k0 = k - H;
-      if (y1) pml_face<R, STAGE>(P.f[1], i0 + (long long)a.nx * ((j - H) + (long long)P.npml * k0), Q, d, ad, by, a.DT, h, false, none);
-      if (y2) pml_face<R, STAGE>(P.f[4], i0 + (long long)a.nx * ((j - H - (a.ny - P.npml)) + (long long)P.npml * k0), Q, d, ad, by, a.DT, h, false, none);
+      if (y1) pml_face<R, STAGE>(P.f[1], i0 + (long long)a.nx * ((j - H) + (long long)P.npml * k0), Q, d, al, by, a.DT, h, false, none);
+      if (y2) pml_face<R, STAGE>(P.f[4], i0 + (long long)a.nx * ((j - H - (a.ny - P.npml)) + (long long)P.npml * k0), Q, d, al, by, a.DT, h, false, none);
     }
   }
   // z: derivatives along zeta (wave_deriv.cpp:234-242)
+  {
+    R f[9][5];
 #pragma unroll
-  for (int v = 0; v < 9; ++v) D[v] = zd(v);
+    for (int v = 0; v < 9; ++v) zt(v, f[v]);
+    cc.load(coef, a, off, 2);
+    bz = P.beta[2][k];
+    loads_issued();
+    diff(FB3, f);
+  }
   assemble(D, cf(M_ZTX), cf(M_ZTY), cf(M_ZTZ), mu, lam, bu, Q);
-  const R bz = P.beta[2][k];
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
     Q[v] *= a.rDH;
@@ -251,10 +329,10 @@ __device__ __forceinline__ void cell_body(const StageArgs<R>& a, const TM* __res
   if (P.npml > 0) {
     const bool z1 = k < H + P.npml, z2 = P.has_z2 && k >= H + a.nz - P.npml;
     if (z1 || z2) {
-      const R d = P.d[2][k], ad = d + P.alpha[2][k];
+      const R d = P.d[2][k], al = P.alpha[2][k];
       const long long i0 = i - H, j0 = j - H;
-      if (z1) pml_face<R, STAGE>(P.f[2], i0 + (long long)a.nx * (j0 + (long long)a.ny * (k - H)), Q, d, ad, bz, a.DT, h, false, none);
-      if (z2) pml_face<R, STAGE>(P.f[5], i0 + (long long)a.nx * (j0 + (long long)a.ny * (k - H - (a.nz - P.npml))), Q, d, ad, bz, a.DT, h, false, none);
+      if (z1) pml_face<R, STAGE>(P.f[2], i0 + (long long)a.nx * (j0 + (long long)a.ny * (k - H)), Q, d, al, bz, a.DT, h, false, none);
+      if (z2) pml_face<R, STAGE>(P.f[5], i0 + (long long)a.nx * (j0 + (long long)a.ny * (k - H - (a.nz - P.npml))), Q, d, al, bz, a.DT, h, false, none);
     }
   }
   // RK4 stage update of W (wave_rk.cpp:18-104). The RK base and stage states
@@ -272,10 +350,10 @@ __device__ __forceinline__ void cell_body(const StageArgs<R>& a, const TM* __res
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
     R* wo = at(a.wout + (long long)v * N, off);
-    if constexpr (STAGE == 0) st_stream(wo, R(wc(v) + R(RK_A2) * h[v]));
+    if constexpr (STAGE == 0) st_stream(wo, R(ctr[v] + R(RK_A2) * h[v]));
     else if constexpr (STAGE == 1) st_stream(wo, R(mv[v] + R(RK_A3) * h[v]));
     else if constexpr (STAGE == 2) st_stream(wo, R(mv[v] + h[v]));
-    else st_stream(wo, rk_close(mv[v], x1[v], x2[v], wc(v), h[v]));
+    else st_stream(wo, rk_close(mv[v], x1[v], x2[v], ctr[v], h[v]));
   }
 }
 
@@ -296,10 +374,12 @@ __global__ __launch_bounds__(256) void cg_cell(StageArgs<R> a, const TM* __restr
   const R* W = a.win;
   cell_body<R, TM, FB1, FB2, FB3, STAGE>(
       a, coef, i, j, k, off,
-      [&](int v) -> R { return mac_off<FB1>(W + (long long)v * N, off, (unsigned)sizeof(R)); },
-      [&](int v) -> R { return mac_off<FB2>(W + (long long)v * N, off, a.rowb); },
-      [&](int v) -> R { return mac_off<FB3>(W + (long long)v * N, off, a.planeb); },
-      [&](int v) -> R { return *at(W + (long long)v * N, off); });
+      [&](int v, R* f) {
+        f[1] = *at(W + (long long)v * N, off);
+        taps_off<FB1>(W + (long long)v * N, off, (unsigned)sizeof(R), f);
+      },
+      [&](int v, R* f) { taps_off<FB2>(W + (long long)v * N, off, a.rowb, f); },
+      [&](int v, R* f) { taps_off<FB3>(W + (long long)v * N, off, a.planeb, f); });
 }
 
 // ---------------------------------------------------------------------------
@@ -375,13 +455,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     }
     cell_body<R, TM, FB1, FB2, FB3, STAGE>(
         a, coef, i, j, k, off,
-        [&](int v) -> R { return mac_off<FB1>(W + (long long)v * N, off, (unsigned)sizeof(R)); },
-        [&](int v) -> R { return mac_off<FB2>(W + (long long)v * N, off, a.rowb); },
-        [&](int v) -> R {
-          return R(FB3) * (R(AF_1) * zw[v][ZL - FB3] + R(AF0) * zw[v][ZL] + R(AF1) * zw[v][ZL + FB3] +
-                           R(AF2) * zw[v][ZL + 2 * FB3] + R(AF3) * zw[v][ZL + 3 * FB3]);
+        [&](int v, R* f) {
+          f[1] = zw[v][ZL];
+          taps_off<FB1>(W + (long long)v * N, off, (unsigned)sizeof(R), f);
         },
-        [&](int v) -> R { return zw[v][ZL]; });
+        [&](int v, R* f) { taps_off<FB2>(W + (long long)v * N, off, a.rowb, f); },
+        [&](int v, R* f) { taps<FB3>(&zw[v][ZL], 1, f); });
 #pragma unroll
     for (int v = 0; v < 9; ++v) {
 #pragma unroll
@@ -460,10 +539,13 @@ __global__ __launch_bounds__(256) void cg_pair(StageArgs<float> a, const float* 
       if (ic < H || ic >= H + a.nx) continue;
       const long long p = (long long)ic + NXl * j + (long long)k * S;
       cell_body<float, float, FB1, FB2, FB3, STAGE>(
-          a, coef, ic, j, k, cell_off(a, ic, j, k), [&](int v) -> float { return mac<FB1>(W + (long long)v * N + p, 1); },
-          [&](int v) -> float { return mac<FB2>(W + (long long)v * N + p, NXl); },
-          [&](int v) -> float { return mac<FB3>(W + (long long)v * N + p, S); },
-          [&](int v) -> float { return W[(long long)v * N + p]; });
+          a, coef, ic, j, k, cell_off(a, ic, j, k),
+          [&](int v, float* f) {
+            f[1] = W[(long long)v * N + p];
+            taps<FB1>(W + (long long)v * N + p, 1, f);
+          },
+          [&](int v, float* f) { taps<FB2>(W + (long long)v * N + p, NXl, f); },
+          [&](int v, float* f) { taps<FB3>(W + (long long)v * N + p, S, f); });
     }
     return;
   }
@@ -634,22 +716,12 @@ __global__ __launch_bounds__(64 * TY) void cg_zcol(StageArgs<R> a, const TM* __r
       const R* L = &sw[buf][0][0];
       cell_body<R, TM, FB1, FB2, FB3, STAGE>(
           a, coef, i, j, k, cell_off(a, i, j, k),
-          [&](int v) -> R {
-            const R* f = L + v * T::LP + cidx;
-            return R(FB1) * (R(AF_1) * f[-FB1] + R(AF0) * f[0] + R(AF1) * f[FB1] + R(AF2) * f[2 * FB1] +
-                             R(AF3) * f[3 * FB1]);
+          [&](int v, R* f) {
+            f[1] = zq[v][ZL];
+            taps<FB1>(L + v * T::LP + cidx, 1, f);
           },
-          [&](int v) -> R {
-            const R* f = L + v * T::LP + cidx;
-            constexpr int s = T::LX;
-            return R(FB2) * (R(AF_1) * f[-FB2 * s] + R(AF0) * f[0] + R(AF1) * f[FB2 * s] +
-                             R(AF2) * f[2 * FB2 * s] + R(AF3) * f[3 * FB2 * s]);
-          },
-          [&](int v) -> R {
-            return R(FB3) * (R(AF_1) * zq[v][ZL - FB3] + R(AF0) * zq[v][ZL] + R(AF1) * zq[v][ZL + FB3] +
-                             R(AF2) * zq[v][ZL + 2 * FB3] + R(AF3) * zq[v][ZL + 3 * FB3]);
-          },
-          [&](int v) -> R { return zq[v][ZL]; });
+          [&](int v, R* f) { taps<FB2>(L + v * T::LP + cidx, T::LX, f); },
+          [&](int v, R* f) { taps<FB3>(&zq[v][ZL], 1, f); });
     }
   }
 }
@@ -693,23 +765,12 @@ __global__ __launch_bounds__(64 * TY) void cg_plane(StageArgs<R> a, const TM* __
   if (!active) return;
   cell_body<R, TM, FB1, FB2, FB3, STAGE>(
       a, coef, i, j, k, cell_off(a, i, j, k),
-      [&](int v) -> R {
-        const R* f = L + v * T::LP + cidx;
-        return R(FB1) * (R(AF_1) * f[-FB1] + R(AF0) * f[0] + R(AF1) * f[FB1] + R(AF2) * f[2 * FB1] +
-                         R(AF3) * f[3 * FB1]);
+      [&](int v, R* f) {
+        f[1] = L[v * T::LP + cidx];
+        taps<FB1>(L + v * T::LP + cidx, 1, f);
       },
-      [&](int v) -> R {
-        const R* f = L + v * T::LP + cidx;
-        constexpr int s = T::LX;
-        return R(FB2) * (R(AF_1) * f[-FB2 * s] + R(AF0) * f[0] + R(AF1) * f[FB2 * s] + R(AF2) * f[2 * FB2 * s] +
-                         R(AF3) * f[3 * FB2 * s]);
-      },
-      [&](int v) -> R {
-        const R* f = W + (long long)v * N + p;
-        return R(FB3) * (R(AF_1) * f[-FB3 * S] + R(AF0) * L[v * T::LP + cidx] + R(AF1) * f[FB3 * S] +
-                         R(AF2) * f[2 * FB3 * S] + R(AF3) * f[3 * FB3 * S]);
-      },
-      [&](int v) -> R { return L[v * T::LP + cidx]; });
+      [&](int v, R* f) { taps<FB2>(L + v * T::LP + cidx, T::LX, f); },
+      [&](int v, R* f) { taps<FB3>(W + (long long)v * N + p, S, f); });
 }
 
 // ---------------------------------------------------------------------------
@@ -821,7 +882,7 @@ __global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __re
   if (in_x1 || in_x2) {
     R Q[9];
     assemble(Dx, cf(M_XIX, p), cf(M_XIY, p), cf(M_XIZ, p), mu, lam, bu, Q);
-    R d = P.d[0][i], ad = d + P.alpha[0][i];
+    R d = P.d[0][i], al = P.alpha[0][i];
     R ex[6] = {0, 0, 0, 0, 0, 0};
     const bool top = (k == ktop);
     if (top) {
@@ -832,13 +893,13 @@ __global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __re
       stress_rows(Vz, cf(M_ZTX, p), cf(M_ZTY, p), cf(M_ZTZ, p), mu, lam, ex);
     }
     long long rowq = (long long)(j - H) + (long long)a.ny * (k - H);
-    if (in_x1) pml_face<R, STAGE>(P.f[0], (long long)(i - H) + (long long)P.npml * rowq, Q, d, ad, bx, a.DT, h, top, ex);
-    if (in_x2) pml_face<R, STAGE>(P.f[3], (long long)(i - H - (a.nx - P.npml)) + (long long)P.npml * rowq, Q, d, ad, bx, a.DT, h, top, ex);
+    if (in_x1) pml_face<R, STAGE>(P.f[0], (long long)(i - H) + (long long)P.npml * rowq, Q, d, al, bx, a.DT, h, top, ex);
+    if (in_x2) pml_face<R, STAGE>(P.f[3], (long long)(i - H - (a.nx - P.npml)) + (long long)P.npml * rowq, Q, d, al, bx, a.DT, h, top, ex);
   }
   if (in_y1 || in_y2) {
     R Q[9];
     assemble(Dy, cf(M_ETX, p), cf(M_ETY, p), cf(M_ETZ, p), mu, lam, bu, Q);
-    R d = P.d[1][j], ad = d + P.alpha[1][j];
+    R d = P.d[1][j], al = P.alpha[1][j];
     R ex[6] = {0, 0, 0, 0, 0, 0};
     const bool top = (k == ktop);
     if (top) {
@@ -849,17 +910,17 @@ __global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __re
       stress_rows(Vz, cf(M_ZTX, p), cf(M_ZTY, p), cf(M_ZTZ, p), mu, lam, ex);
     }
     long long i0 = i - H, k0 = k - H;
-    if (in_y1) pml_face<R, STAGE>(P.f[1], i0 + (long long)a.nx * ((j - H) + (long long)P.npml * k0), Q, d, ad, by, a.DT, h, top, ex);
-    if (in_y2) pml_face<R, STAGE>(P.f[4], i0 + (long long)a.nx * ((j - H - (a.ny - P.npml)) + (long long)P.npml * k0), Q, d, ad, by, a.DT, h, top, ex);
+    if (in_y1) pml_face<R, STAGE>(P.f[1], i0 + (long long)a.nx * ((j - H) + (long long)P.npml * k0), Q, d, al, by, a.DT, h, top, ex);
+    if (in_y2) pml_face<R, STAGE>(P.f[4], i0 + (long long)a.nx * ((j - H - (a.ny - P.npml)) + (long long)P.npml * k0), Q, d, al, by, a.DT, h, top, ex);
   }
   if (in_z1) {  // only for very shallow grids: bottom PML reaching the surface layers
     R Dz[9], Q[9];
 #pragma unroll
     for (int v = 0; v < 9; ++v) Dz[v] = mac<FB3>(W + (long long)v * N + p, S) * a.rDH;
     assemble(Dz, cf(M_ZTX, p), cf(M_ZTY, p), cf(M_ZTZ, p), mu, lam, bu, Q);
-    R d = P.d[2][k], ad = d + P.alpha[2][k], bz = P.beta[2][k];
+    R d = P.d[2][k], al = P.alpha[2][k], bz = P.beta[2][k];
     const R none[6] = {0, 0, 0, 0, 0, 0};
-    pml_face<R, STAGE>(P.f[2], (long long)(i - H) + (long long)a.nx * ((j - H) + (long long)a.ny * (k - H)), Q, d, ad, bz, a.DT, h, false, none);
+    pml_face<R, STAGE>(P.f[2], (long long)(i - H) + (long long)a.nx * ((j - H) + (long long)a.ny * (k - H)), Q, d, al, bz, a.DT, h, false, none);
   }
   // RK4 stage update: every load before the first store (see cell_body)
   R out[9], mv[9], x1[9], x2[9], x3[9];
