@@ -103,38 +103,57 @@ struct SolverBase {
   // pNX is the device row pitch, pXe the padded x extent (nx + 6)
   int pNX = 0, pNY = 0, pNZ = 0, pXe = 0;
 
-  // Strided device-to-host copy of the interior of one padded plane of a
-  // plane-major array (x fastest): axis 0 = the y-z plane at i = index
-  // ([nz][ny]), 1 = the x-z plane at j = index ([nz][nx]), 2 = the x-y plane at
-  // k = index ([ny][nx]). No kernel: hipMemcpy2D with the plane's stride.
+  // Staging buffer of the getters and setters, part of the solver: rows are packed
+  // into it on the device (launch_gather) and copied in one piece, STAGE bytes at a
+  // time; a row always fits.
+  static constexpr long long STAGE = 32LL << 20;
+  double* stage = nullptr;
+  long long stage_n = 0;  // doubles
+  int alloc_stage() {
+    const long long tN = (long long)pXe * pNY * pNZ;
+    stage_n = std::max(std::min(tN, STAGE / 8), (long long)std::max(pXe, std::max(pNY, pNZ)));
+    return dalloc(&stage, stage_n);
+  }
+  // `rows` rows of `na` elements, sa apart, a row every sb elements, to host as X
+  template <class T, class X>
+  int gather(const T* src, long long sa, long long sb, int na, long long rows, X* host, double sc) {
+    const long long step = std::max(1LL, stage_n * 8 / (long long)sizeof(X) / na);
+    for (long long r = 0; r < rows; r += step) {
+      const long long m = std::min(step, rows - r);
+      cg::launch_gather<T, X>(src + r * sb, sa, sb, na, m, reinterpret_cast<X*>(stage), sc, stream);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipMemcpyAsync(host + r * na, stage, sizeof(X) * m * na, hipMemcpyDeviceToHost, stream));
+    }
+    HIPCHK(hipStreamSynchronize(stream));
+    return CGFDM_OK;
+  }
+  // the same without conversion
+  template <class T>
+  int gather_raw(const T* src, long long sa, long long sb, int na, long long rows, T* host) {
+    using W = typename std::conditional<sizeof(T) == 2, unsigned short,
+                                        typename std::conditional<sizeof(T) == 4, unsigned, unsigned long long>::type>::type;
+    return gather(reinterpret_cast<const W*>(src), sa, sb, na, rows, reinterpret_cast<W*>(host), 1.0);
+  }
+
+  // Interior of one padded plane of a plane-major array (x fastest): axis 0 = the
+  // y-z plane at i = index ([nz][ny]), 1 = the x-z plane at j = index ([nz][nx]),
+  // 2 = the x-y plane at k = index ([ny][nx]); strides and offset of its rows.
+  struct PlaneRows {
+    long long first, sa, sb;
+    int na, nb;
+  };
+  PlaneRows plane_rows(int axis, int index) const {
+    const int H = 3;
+    const long long S2 = (long long)pNX * pNY;
+    if (axis == 0) return {index + (long long)pNX * H + S2 * H, pNX, S2, pNY - 2 * H, pNZ - 2 * H};
+    if (axis == 1) return {H + (long long)pNX * index + S2 * H, 1, S2, pXe - 2 * H, pNZ - 2 * H};
+    return {H + (long long)pNX * H + S2 * index, 1, pNX, pXe - 2 * H, pNY - 2 * H};
+  }
   template <class T>
   int copy_plane(const T* plane0, int axis, int index, std::vector<T>& out) {
-    const int H = 3;
-    const size_t e = sizeof(T);
-    const long long S2 = (long long)pNX * pNY;
-    int na, nb;
-    if (axis == 0) {
-      na = pNY - 2 * H;
-      nb = pNZ - 2 * H;
-      out.resize((size_t)na * nb);
-      // one element per padded row, rows j = H.. of planes k = H..
-      for (int b = 0; b < nb; ++b)
-        HIPCHK(hipMemcpy2D(out.data() + (size_t)b * na, e, plane0 + index + (long long)pNX * H + S2 * (b + H),
-                           e * pNX, e, na, hipMemcpyDeviceToHost));
-    } else if (axis == 1) {
-      na = pXe - 2 * H;
-      nb = pNZ - 2 * H;
-      out.resize((size_t)na * nb);
-      HIPCHK(hipMemcpy2D(out.data(), e * na, plane0 + H + (long long)pNX * index + S2 * H, e * S2, e * na, nb,
-                         hipMemcpyDeviceToHost));
-    } else {
-      na = pXe - 2 * H;
-      nb = pNY - 2 * H;
-      out.resize((size_t)na * nb);
-      HIPCHK(hipMemcpy2D(out.data(), e * na, plane0 + H + (long long)pNX * H + S2 * index, e * pNX, e * na, nb,
-                         hipMemcpyDeviceToHost));
-    }
-    return CGFDM_OK;
+    const PlaneRows p = plane_rows(axis, index);
+    out.resize((size_t)p.na * p.nb);
+    return gather_raw(plane0 + p.first, p.sa, p.sb, p.na, p.nb, out.data());
   }
   // Rows of pXe elements between the tight layout of the C ABI (pitch pXe)
   // and the device layout (pitch pNX); strided hipMemcpy2D, no kernel.
@@ -149,19 +168,26 @@ struct SolverBase {
                               stream));
     return CGFDM_OK;
   }
-  // `planes` device volumes to / from a tight host array
+  // a device volume to a tight host array
   template <class X>
-  int to_host(const X* dev, X* host, int planes) {
-    const size_t e = sizeof(X);
-    HIPCHK(hipStreamSynchronize(stream));
-    HIPCHK(hipMemcpy2D(host, e * pXe, dev, e * pNX, e * pXe, (size_t)planes * pNY * pNZ, hipMemcpyDeviceToHost));
-    return CGFDM_OK;
+  int to_host(const X* dev, X* host) {
+    return gather_raw(dev, 1, pNX, pXe, (long long)pNY * pNZ, host);
   }
-  template <class X>
-  int to_dev(X* dev, const X* host, int planes) {
-    const size_t e = sizeof(X);
+  // a device volume to / from a tight host array of doubles, times sc
+  template <class T>
+  int volume_out(const T* dev, double* host, double sc) {
+    return gather(dev, 1, pNX, pXe, (long long)pNY * pNZ, host, sc);
+  }
+  template <class T>
+  int volume_in(T* dev, const double* host, double sc) {
+    const long long rows = (long long)pNY * pNZ, step = std::max(1LL, stage_n / pXe);
+    for (long long r = 0; r < rows; r += step) {
+      const long long m = std::min(step, rows - r);
+      HIPCHK(hipMemcpyAsync(stage, host + r * pXe, sizeof(double) * m * pXe, hipMemcpyHostToDevice, stream));
+      cg::launch_scatter<T>(dev + r * pNX, pNX, pXe, m, stage, sc, stream);
+      HIPCHK(hipGetLastError());
+    }
     HIPCHK(hipStreamSynchronize(stream));
-    HIPCHK(hipMemcpy2D(dev, e * pNX, host, e * pXe, e * pXe, (size_t)planes * pNY * pNZ, hipMemcpyHostToDevice));
     return CGFDM_OK;
   }
   // tight linear cell index -> device cell index (-1 outside the interior)
@@ -508,6 +534,7 @@ struct Solver : SolverBase {
     pNY = NY;
     pNZ = NZ;
     pXe = tNX;
+    if ((rc = alloc_stage())) return rc;
     if constexpr (kPacked16) {
       unsigned* words = nullptr;
       if ((rc = galloc(&words, (long long)(cg::M_NCOEF / 2) * N))) return rc;
@@ -847,30 +874,18 @@ struct Solver : SolverBase {
 
   int get_field(int comp, double* out) override {
     if (comp < 0 || comp > 8) return fail(CGFDM_ERR_ARG, "component out of range");
-    std::vector<R> h(tN);
-    if (int rc = to_host(A + (size_t)comp * N, h.data(), 1)) return rc;
-    double sc = comp >= 3 ? Z : 1.0;
-    for (long long p = 0; p < tN; ++p) out[p] = (double)h[p] * sc;
-    return CGFDM_OK;
+    return volume_out(A + (size_t)comp * N, out, comp >= 3 ? Z : 1.0);
   }
 
   int get_slice(int comp, int axis, int index, float* out) override {
     if (int rc = check_plane(comp, axis, index)) return rc;
-    HIPCHK(hipStreamSynchronize(stream));
-    std::vector<R> h;
-    if (int rc = copy_plane(A + (size_t)comp * N, axis, index, h)) return rc;
-    const double sc = comp >= 3 ? Z : 1.0;
-    for (size_t p = 0; p < h.size(); ++p) out[p] = (float)((double)h[p] * sc);
-    return CGFDM_OK;
+    const PlaneRows p = plane_rows(axis, index);
+    return gather(A + (size_t)comp * N + p.first, p.sa, p.sb, p.na, p.nb, out, comp >= 3 ? Z : 1.0);
   }
 
   int set_field(int comp, const double* in) override {
     if (comp < 0 || comp > 8) return fail(CGFDM_ERR_ARG, "component out of range");
-    HIPCHK(hipStreamSynchronize(stream));
-    std::vector<R> h(tN);
-    double sc = comp >= 3 ? 1.0 / Z : 1.0;
-    for (long long p = 0; p < tN; ++p) h[p] = R(in[p] * sc);
-    return to_dev(A + (size_t)comp * N, h.data(), 1);
+    return volume_in(A + (size_t)comp * N, in, comp >= 3 ? 1.0 / Z : 1.0);
   }
 
   int get_setup(int what, double* out) override {
@@ -879,7 +894,7 @@ struct Solver : SolverBase {
       const int plane = what < 9 ? what : what - 1;
       std::vector<unsigned> h(tN);
       std::vector<float> ha(2 * (size_t)cg::M_NCOEF * NZ);
-      if (int rc = to_host(reinterpret_cast<const unsigned*>(coef) + (size_t)(plane >> 1) * N, h.data(), 1)) return rc;
+      if (int rc = to_host(reinterpret_cast<const unsigned*>(coef) + (size_t)(plane >> 1) * N, h.data())) return rc;
       HIPCHK(hipMemcpy(ha.data(), aff, sizeof(float) * ha.size(), hipMemcpyDeviceToHost));
       const double sc = what == 10 || what == 11 ? Z : what == 12 ? 1.0 / Z : 1.0;
       for (long long p = 0; p < tN; ++p) {
@@ -893,7 +908,7 @@ struct Solver : SolverBase {
     if (what >= 0 && what <= 12 && what != 9) {
       int plane = what < 9 ? what : what - 1;  // 10,11,12 -> M_MU.. (9,10,11)
       std::vector<TM> h(tN);
-      if (int rc = to_host(coef + (size_t)plane * N, h.data(), 1)) return rc;
+      if (int rc = to_host(coef + (size_t)plane * N, h.data())) return rc;
       double sc = what == 10 || what == 11 ? Z : what == 12 ? 1.0 / Z : 1.0;
       for (long long p = 0; p < tN; ++p) {
         double v = sizeof(TM) == 8 ? (double)*(const double*)(const void*)&h[p] : (double)to_float(h[p]);
@@ -902,10 +917,7 @@ struct Solver : SolverBase {
       return CGFDM_OK;
     }
     if (what == 9) {
-      std::vector<R> h(tN);
-      if (int rc = to_host(jac, h.data(), 1)) return rc;
-      for (long long p = 0; p < tN; ++p) out[p] = (double)h[p];
-      return CGFDM_OK;
+      return volume_out(jac, out, 1.0);
     }
     if ((what >= 20 && what < 29) || (what >= 30 && what < 39)) {
       const R* src = (what < 30 ? rdzdx : rdzdy) + (size_t)(what % 10) * S;
@@ -1414,6 +1426,7 @@ struct AwenoSolver : SolverBase {
     pNY = NY;
     pNZ = NZ;
     pXe = tNX;
+    if ((rc = alloc_stage())) return rc;
     if ((rc = galloc(&cjm, (long long)aw::C_N * N))) return rc;
     if ((rc = repack(cjm, cjm_t, (long long)aw::C_N * NY * NZ, true))) return rc;
     HIPCHK(hipStreamSynchronize(stream));
@@ -1612,10 +1625,7 @@ struct AwenoSolver : SolverBase {
 
   int get_field(int comp, double* out) override {
     if (comp < 0 || comp > 8) return fail(CGFDM_ERR_ARG, "component out of range");
-    std::vector<R> h(tN);
-    if (int rc = to_host(buf[cur] + (size_t)comp * N, h.data(), 1)) return rc;
-    for (long long p = 0; p < tN; ++p) out[p] = (double)h[p];
-    return CGFDM_OK;
+    return volume_out(buf[cur] + (size_t)comp * N, out, 1.0);
   }
 
   // physical (Vx, Vy, Vz, Txx, Tyy, Tzz, Txy, Txz, Tyz) from the conservative
@@ -1623,7 +1633,6 @@ struct AwenoSolver : SolverBase {
   // data_io.cpp:435-483)
   int get_slice(int comp, int axis, int index, float* out) override {
     if (int rc = check_plane(comp, axis, index)) return rc;
-    HIPCHK(hipStreamSynchronize(stream));
     const R* W = buf[cur];
     std::vector<R> u0, u1, u2, mu, lam, b;
     int rc;
@@ -1656,10 +1665,7 @@ struct AwenoSolver : SolverBase {
 
   int set_field(int comp, const double* in) override {
     if (comp < 0 || comp > 8) return fail(CGFDM_ERR_ARG, "component out of range");
-    HIPCHK(hipStreamSynchronize(stream));
-    std::vector<R> h(tN);
-    for (long long p = 0; p < tN; ++p) h[p] = R(in[p]);
-    if (int rc = to_dev(buf[cur] + (size_t)comp * N, h.data(), 1)) return rc;
+    if (int rc = volume_in(buf[cur] + (size_t)comp * N, in, 1.0)) return rc;
     // the marching stages leave the ghost cells of their output buffers alone
     if (march)
       for (int q = 1; q < 3; ++q)
@@ -1670,10 +1676,7 @@ struct AwenoSolver : SolverBase {
 
   int get_setup(int what, double* out) override {
     if (what < 0 || what >= aw::C_N) return fail(CGFDM_ERR_ARG, "unknown setup product");
-    std::vector<R> h(tN);
-    if (int rc = to_host(cjm + (size_t)what * N, h.data(), 1)) return rc;
-    for (long long p = 0; p < tN; ++p) out[p] = (double)h[p];
-    return CGFDM_OK;
+    return volume_out(cjm + (size_t)what * N, out, 1.0);
   }
 };
 

@@ -25,6 +25,14 @@ void launch_hrange(const float* coord, double* part, int nblocks, int nx, int ny
                    hipStream_t st);
 void launch_frange(const float* a, long long n, double* part, int nblocks, hipStream_t st);
 
+// Rows of `na` elements, sa elements apart, one row every sb elements, packed into
+// `out` as X = sc * value (gather), or spread from `in` (scatter).
+template <class T, class X>
+void launch_gather(const T* src, long long sa, long long sb, int na, long long rows, X* out, double sc,
+                   hipStream_t st);
+template <class T>
+void launch_scatter(T* dst, long long sb, int na, long long rows, const double* in, double sc, hipStream_t st);
+
 // Allocation-free CFL ranges of a device-resident grid: per-block partials in a
 // library-owned 64 KiB device array (RANGE_BLOCKS pairs per reduction), the
 // eight results written to the device array out8. Asynchronous on st.

@@ -78,3 +78,20 @@ def test_slice_rejects_out_of_range():
     for comp, axis, idx in ((9, 0, H), (0, 3, H), (0, 0, H - 1), (0, 0, H + m.nx), (0, 2, H + m.nz)):
         with pytest.raises(Exception):
             g.slice(comp, axis, idx)
+
+
+def test_fields_and_slices_of_a_grid_larger_than_one_copy():
+    """Fields go to and from the device in pieces of 32 MB: a grid of two pieces, the second one partial, keeps
+    every value (exactly: they are stored in 32 bits), and its slices are planes of the field."""
+    from cgfdm_amd import solver
+    nx, ny, nz = 190, 170, 140
+    m = M.small_config(nx=nx, ny=ny, nz=nz, npml=0, hills=0, layered=False)
+    g = solver.Solver(m, precision=4)
+    assert g.N * 8 > 32 << 20
+    want = np.random.default_rng(5).standard_normal(g.shape).astype(np.float32)
+    for c in (1, 4):
+        print(f"field {c} of {nx}x{ny}x{nz}", flush=True)
+        g.set_field(c, want)
+        np.testing.assert_array_equal(g.field(c), want)
+        for axis, idx, sl in planes(nz, ny, nx):
+            np.testing.assert_array_equal(g.slice(c, axis, idx), want[sl])
