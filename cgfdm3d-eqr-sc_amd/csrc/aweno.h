@@ -28,7 +28,7 @@ struct StageArgs {
 template <class R>
 void launch_faces(const StageArgs<R>& a, hipStream_t st);
 template <class R>
-void launch_update(const StageArgs<R>& a, int nx, int ny, hipStream_t st, hipStream_t st_top);
+void launch_update(const StageArgs<R>& a, int nx, int ny, hipStream_t st);
 // The stage in two marching kernels without the flux array (aweno_march.h): y
 // first, then x, z and the top layers.
 void launch_march_y(const StageArgs<float>& a, int nx, int ny, hipStream_t st);

@@ -356,18 +356,6 @@ float bits16_to_float(unsigned short) { return 0.f; }
 template <class R, class TM>
 struct Solver : SolverBase {
   cgfdm_desc d{};
-  // surface stage kernels on a second stream, forked from and joined to the
-  // solver's stream around every stage (CGFDM_SURFACE_STREAM=0: one stream):
-  // they write only the top three layers, which the interior kernel of the
-  // same stage neither writes nor reads, so the two run side by side
-  int surf_overlap = 1;
-  hipStream_t sstream = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  ~Solver() override {
-    if (ev_fork) (void)hipEventDestroy(ev_fork);
-    if (ev_join) (void)hipEventDestroy(ev_join);
-    if (sstream) (void)hipStreamDestroy(sstream);
-  }
   // device layout: row pitch NX (nx + 6 rounded up to 32 elements in the
   // row-aligned layout), plane S = NX NY, volume N = S NZ; the host-facing
   // arrays of the C ABI use the tight layout tNX = nx + 6 (tS, tN)
@@ -460,7 +448,6 @@ struct Solver : SolverBase {
     }
     if (const char* e = std::getenv("CGFDM_INTERIOR_ZTY")) zty = std::atoi(e) == 4 ? 4 : 8;
     if (const char* e = std::getenv("CGFDM_ADJOINT_PIPE")) adj_pipe = std::atoi(e) != 0 ? 1 : 0;
-    if (const char* e = std::getenv("CGFDM_SURFACE_STREAM")) surf_overlap = std::atoi(e) != 0 ? 1 : 0;
     if (const char* e = std::getenv("CGFDM_INTERIOR_ZREG")) {
       const int v = std::atoi(e);
       if (v >= 0 && v <= 4096) zreg = v;
@@ -747,17 +734,17 @@ struct Solver : SolverBase {
     return zreg > 0 ? "cg_zreg" : "cg_cell";
   }
 
+  int launch_stage(const cg::StageArgs<R>& a, const cg::SurfArgs<R>& sa, const int (&fb)[3]) {
+    if (d.free_surface) LAUNCHCHK((cg::launch_stage<R, TM>(a, coef, sa, fb[0], fb[1], fb[2], stream)), "stage");
+    else LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
+    return CGFDM_OK;
+  }
+
   // observe = false: no station record, PGV or displacement update (used to
   // recompute states for the adjoint)
   int step_impl(int n, bool observe) {
     if (!kCgfdmStepEnabled) return fail(CGFDM_ERR_DISABLED, kCgfdmStepOff);
     const int kend = cg::H + d.nz - (d.free_surface ? 3 : 0);
-    const bool fork = d.free_surface && surf_overlap;
-    if (fork && !sstream) {
-      HIPCHK(hipStreamCreateWithFlags(&sstream, hipStreamNonBlocking));
-      HIPCHK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-      HIPCHK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
-    }
     for (int s = 0; s < n; ++s) {
       int fb[3] = {FBTAB[it % 8][0], FBTAB[it % 8][1], FBTAB[it % 8][2]};
       size_t sp = 0;
@@ -806,32 +793,25 @@ struct Solver : SolverBase {
         a.x1 = B;
         a.x2 = C;
         a.pml = pml;
-        // the surface stage (forked first, so that its few blocks are
-        // dispatched before the interior's) and the interior stage
-        if (d.free_surface) {
-          hipStream_t ss = fork ? sstream : stream;
-          if (fork) {
-            HIPCHK(hipEventRecord(ev_fork, stream));
-            HIPCHK(hipStreamWaitEvent(sstream, ev_fork, 0));
+        // the surface and the interior stage on one stream: they may run side by
+        // side, but the events that fork and join a second stream cost more (us per
+        // step: 24 x 20 x 16 146 -> 95, 128 x 128 x 64 321 -> 286, 512 x 512 x 256
+        // 14014 -> 14033). With timing on, each is launched and timed by itself.
+        cg::SurfArgs<R> sa{jac, rdzdx, rdzdy, observe ? pgv : nullptr, dis};
+        if (!timing_on) {
+          if (int rc = launch_stage(a, sa, fb)) return rc;
+        } else {
+          if (d.free_surface) {
+            const size_t fp = next_pair(1);
+            HIPCHK(hipEventRecord(ev[fp].a, stream));
+            LAUNCHCHK((cg::launch_surface<R, TM>(a, coef, sa, fb[0], fb[1], fb[2], stream)), "surface stage");
+            HIPCHK(hipEventRecord(ev[fp].b, stream));
           }
-          cg::SurfArgs<R> sa{jac, rdzdx, rdzdy, observe ? pgv : nullptr, dis};
-          size_t fp = 0;
-          if (timing_on) {
-            fp = next_pair(1);
-            HIPCHK(hipEventRecord(ev[fp].a, ss));
-          }
-          LAUNCHCHK((cg::launch_surface<R, TM>(a, coef, sa, fb[0], fb[1], fb[2], ss)), "surface stage");
-          if (timing_on) HIPCHK(hipEventRecord(ev[fp].b, ss));
-          if (fork) HIPCHK(hipEventRecord(ev_join, sstream));
-        }
-        size_t ip = 0;
-        if (timing_on) {
-          ip = next_pair(0);
+          const size_t ip = next_pair(0);
           HIPCHK(hipEventRecord(ev[ip].a, stream));
+          LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
+          HIPCHK(hipEventRecord(ev[ip].b, stream));
         }
-        LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
-        if (timing_on) HIPCHK(hipEventRecord(ev[ip].b, stream));
-        if (fork) HIPCHK(hipStreamWaitEvent(stream, ev_join, 0));
         fb[0] = -fb[0];
         fb[1] = -fb[1];
         fb[2] = -fb[2];
@@ -1066,11 +1046,7 @@ struct Solver : SolverBase {
       a.kbeg = cg::H; a.kend = kend; a.stage = irk; a.rty = rty; a.rtx = rtx; a.zreg = zreg; a.kc = kc; a.zty = zty;
       a.DT = R(d.dt); a.rDH = R(1.0 / d.dh); a.aff = aff; a.nzp = NZ;
       a.win = ins[irk]; a.wout = outs[irk]; a.wm = x0; a.x1 = x1; a.x2 = x2; a.pml = pml;
-      LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
-      if (d.free_surface) {
-        cg::SurfArgs<R> sa{jac, rdzdx, rdzdy, observe ? pgv : nullptr, dis};
-        LAUNCHCHK((cg::launch_surface<R, TM>(a, coef, sa, fb[0], fb[1], fb[2], stream)), "surface stage");
-      }
+      if (int rc = launch_stage(a, cg::SurfArgs<R>{jac, rdzdx, rdzdy, observe ? pgv : nullptr, dis}, fb)) return rc;
       fb[0] = -fb[0]; fb[1] = -fb[1]; fb[2] = -fb[2];
     }
     ++it;
@@ -1103,11 +1079,7 @@ struct Solver : SolverBase {
       a.kbeg = cg::H; a.kend = kend; a.stage = irk; a.rty = rty; a.rtx = rtx; a.zreg = zreg; a.kc = kc; a.zty = zty;
       a.DT = R(d.dt); a.rDH = R(1.0 / d.dh); a.aff = aff; a.nzp = NZ;
       a.win = ins[irk]; a.wout = outs[irk]; a.wm = A; a.x1 = B; a.x2 = C; a.pml = pml;
-      LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
-      if (d.free_surface) {
-        cg::SurfArgs<R> sa{jac, rdzdx, rdzdy, nullptr, dis};
-        LAUNCHCHK((cg::launch_surface<R, TM>(a, coef, sa, fb[0], fb[1], fb[2], stream)), "surface stage");
-      }
+      if (int rc = launch_stage(a, cg::SurfArgs<R>{jac, rdzdx, rdzdy, nullptr, dis}, fb)) return rc;
       fb[0] = -fb[0]; fb[1] = -fb[1]; fb[2] = -fb[2];
     }
     return CGFDM_OK;
@@ -1328,16 +1300,6 @@ struct Solver : SolverBase {
 template <class R>
 struct AwenoSolver : SolverBase {
   cgfdm_desc d{};
-  // the top-layer update on a second stream beside the bulk update, forked
-  // from and joined to the solver's stream (CGFDM_SURFACE_STREAM=0: one stream)
-  int surf_overlap = 1;
-  hipStream_t sstream = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  ~AwenoSolver() override {
-    if (ev_fork) (void)hipEventDestroy(ev_fork);
-    if (ev_join) (void)hipEventDestroy(ev_join);
-    if (sstream) (void)hipStreamDestroy(sstream);
-  }
   // device layout (row pitch NX) and the tight layout of the C ABI (tNX), as
   // in the CGFDM solver
   int NX = 0, NY = 0, NZ = 0;
@@ -1381,7 +1343,6 @@ struct AwenoSolver : SolverBase {
       const int v = std::atoi(e);
       if (v >= 0 && v <= 64) rtx = v;
     }
-    if (const char* e = std::getenv("CGFDM_SURFACE_STREAM")) surf_overlap = std::atoi(e) != 0 ? 1 : 0;
     if (const char* e = std::getenv("CGFDM_ROW_ALIGN")) galign = std::atoi(e) != 0;
     tNX = d.nx + 2 * cg::H;
     NX = tNX;
@@ -1509,11 +1470,6 @@ struct AwenoSolver : SolverBase {
   }
 
   int step(int n) override {
-    if (surf_overlap && !march && !sstream) {
-      HIPCHK(hipStreamCreateWithFlags(&sstream, hipStreamNonBlocking));
-      HIPCHK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-      HIPCHK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
-    }
     for (int s = 0; s < n; ++s) {
       size_t sp = 0;
       if (timing_on) {
@@ -1575,16 +1531,8 @@ struct AwenoSolver : SolverBase {
           if (timing_on) HIPCHK(hipEventRecord(ev[up].b, stream));
           continue;
         }
-        if (surf_overlap) {
-          HIPCHK(hipEventRecord(ev_fork, stream));
-          HIPCHK(hipStreamWaitEvent(sstream, ev_fork, 0));
-        }
-        aw::launch_update<R>(a, d.nx, d.ny, stream, surf_overlap ? sstream : stream);
+        aw::launch_update<R>(a, d.nx, d.ny, stream);
         if (timing_on) HIPCHK(hipEventRecord(ev[up].b, stream));
-        if (surf_overlap) {
-          HIPCHK(hipEventRecord(ev_join, sstream));
-          HIPCHK(hipStreamWaitEvent(stream, ev_join, 0));
-        }
       }
       cur = o1;
       W = buf[cur];

@@ -362,9 +362,9 @@ __device__ __forceinline__ void cell_body(const StageArgs<R>& a, const TM* __res
 // ---------------------------------------------------------------------------
 
 template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
-__global__ __launch_bounds__(256) void cg_cell(StageArgs<R> a, const TM* __restrict__ coef) {
+__device__ __forceinline__ void cell_block(const StageArgs<R>& a, const TM* __restrict__ coef, int block) {
   CellTile t;
-  if (!interior_tile(blockIdx.x, a.nx, a.ny, a.kend - a.kbeg, a.rtx, a.rty, t)) return;
+  if (!interior_tile(block, a.nx, a.ny, a.kend - a.kbeg, a.rtx, a.rty, t)) return;
   const int i = H + t.i0 + (threadIdx.x & 63);
   const int j = H + t.j0 + (threadIdx.x >> 6);
   const int k = a.kbeg + t.k;
@@ -380,6 +380,11 @@ __global__ __launch_bounds__(256) void cg_cell(StageArgs<R> a, const TM* __restr
       },
       [&](int v, R* f) { taps_off<FB2>(W + (long long)v * N, off, a.rowb, f); },
       [&](int v, R* f) { taps_off<FB3>(W + (long long)v * N, off, a.planeb, f); });
+}
+
+template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
+__global__ __launch_bounds__(256) void cg_cell(StageArgs<R> a, const TM* __restrict__ coef) {
+  cell_block<R, TM, FB1, FB2, FB3, STAGE>(a, coef, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -777,11 +782,12 @@ __global__ __launch_bounds__(64 * TY) void cg_plane(StageArgs<R> a, const TM* __
 // surface kernel: top three layers, traction image
 // ---------------------------------------------------------------------------
 template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
-__global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __restrict__ coef, SurfArgs<R> s) {
-  const int i = H + blockIdx.x * 64 + (threadIdx.x & 63);
-  const int j = H + blockIdx.y * 4 + (threadIdx.x >> 6);
+__device__ __forceinline__ void surface_block(const StageArgs<R>& a, const TM* __restrict__ coef, const SurfArgs<R>& s,
+                                              int tile_x, int tile_y, int depth) {
+  const int i = H + tile_x * 64 + (threadIdx.x & 63);
+  const int j = H + tile_y * 4 + (threadIdx.x >> 6);
   const int ktop = H + a.nz - 1;
-  const int k = ktop - blockIdx.z;  // blockIdx.z = 0,1,2 -> surface, one below, two below
+  const int k = ktop - depth;  // depth = 0,1,2 -> surface, one below, two below
   if (i >= H + a.nx || j >= H + a.ny) return;
   const long long N = a.N, S = a.S, NXl = a.NX;
   const long long p = (long long)i + NXl * j + (long long)k * S;
@@ -954,6 +960,21 @@ __global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __re
     s.dis[SS + sp] += out[1] * a.DT;
     s.dis[2 * SS + sp] += out[2] * a.DT;
   }
+}
+
+template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
+__global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __restrict__ coef, SurfArgs<R> s) {
+  surface_block<R, TM, FB1, FB2, FB3, STAGE>(a, coef, s, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// Both in one launch, the surface blocks first, for grids whose blocks are all
+// resident at once (launch_stage): there the two kernels are bound by the latency
+// of their loads, one after the other, and registers for more waves have no use.
+template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
+__global__ __launch_bounds__(256) void cg_stage(StageArgs<R> a, const TM* __restrict__ coef, SurfArgs<R> s) {
+  const int ntx = (a.nx + 63) / 64, nty = (a.ny + 3) / 4, b = blockIdx.x, n = 3 * ntx * nty;
+  if (b < n) surface_block<R, TM, FB1, FB2, FB3, STAGE>(a, coef, s, b % ntx, b / ntx % nty, b / (ntx * nty));
+  else cell_block<R, TM, FB1, FB2, FB3, STAGE>(a, coef, b - n);
 }
 
 // ---------------------------------------------------------------------------

@@ -4,6 +4,7 @@
 namespace cg {
 template int launch_interior<float, float>(StageArgs<float>, const float*, int, int, int, hipStream_t);
 template int launch_surface<float, float>(StageArgs<float>, const float*, SurfArgs<float>, int, int, int, hipStream_t);
+template int launch_stage<float, float>(StageArgs<float>, const float*, SurfArgs<float>, int, int, int, hipStream_t);
 }  // namespace cg
 
 namespace cg {

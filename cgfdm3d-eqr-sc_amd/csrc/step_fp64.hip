@@ -4,6 +4,7 @@
 namespace cg {
 template int launch_interior<double, double>(StageArgs<double>, const double*, int, int, int, hipStream_t);
 template int launch_surface<double, double>(StageArgs<double>, const double*, SurfArgs<double>, int, int, int, hipStream_t);
+template int launch_stage<double, double>(StageArgs<double>, const double*, SurfArgs<double>, int, int, int, hipStream_t);
 }  // namespace cg
 
 namespace cg {

@@ -49,3 +49,25 @@ def test_variant_matches_oracle(scheme, var, val, monkeypatch, oracle_mod):
         assert err < 3e-5, (scheme, var, val, v, err)
     sg, so = g.stations(), o.stations()
     assert rel_l2(sg, so) < 3e-5
+
+
+# One launch per stage for grids of at most 1024 blocks, two for larger ones, the
+# interior's last eight regions cut into eighths: grids on both sides of the line,
+# with whole and partial tiles and region counts of 2, 5, 8 and 13.
+@pytest.mark.parametrize("nx,ny,nz", [(24, 16, 12), (70, 40, 20), (66, 60, 40), (130, 100, 26)])
+@pytest.mark.parametrize("coef", [0, 1])
+def test_stage_launches_match_oracle(nx, ny, nz, coef, oracle_mod):
+    from cgfdm_amd import model as M
+    from cgfdm_amd import solver
+    m = M.small_config(nx=nx, ny=ny, nz=nz, npml=4, hills=2, layered=True, free_surface=True, nt=8)
+    print(f"{nx}x{ny}x{nz} coef {coef}, FP32, 8 steps", flush=True)
+    g = solver.Solver(m, precision=4, coef_storage=coef)
+    o = oracle_mod.Oracle(m, prec=4, threads=8)
+    g.step(8)
+    g.synchronize()
+    o.step(8)
+    # FP32: as above; fp16 storage: the rounding of the coefficients, 2^-11 of a layer's range, over 8 steps
+    tol = 3e-5 if coef == 0 else 5e-3
+    for v in range(9):
+        err = rel_l2(g.field(v), o.field(v))
+        assert err < tol, (nx, ny, nz, coef, v, err)
