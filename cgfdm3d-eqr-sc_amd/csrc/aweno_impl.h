@@ -16,66 +16,17 @@ namespace aw {
 
 using cg::H;
 
-// Reciprocal used for the WENO weights: the hardware reciprocal (1 ulp) in
-// FP32, an exact division in FP64.
-__device__ __forceinline__ float wrcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double wrcp(double x) { return 1.0 / x; }
-
-// WENO5-JS value at x_{i+1/2} from u1..u5 = u(i-2..i+2)
-// (alternative_flux_FD.cpp:43-59). The smoothness indicators are written as
-// the sums of squares they expand to, e.g. (10 u3^2 - 31 u3 u4 + 25 u4^2 +
-// 11 u3 u5 - 19 u4 u5 + 4 u5^2) / 3 = 13/12 (u3 - 2 u4 + u5)^2 +
-// 1/4 (3 u3 - 4 u4 + u5)^2; the weights are d_k / (beta_k + 1e-6)^2 with
-// d = (5/16, 10/16, 1/16), normalised.
-template <class R>
-__device__ __forceinline__ R weno5(R u1, R u2, R u3, R u4, R u5) {
-  // the reference scales the expanded form by the literal 0.3333333333, i.e.
-  // the sums of squares by 0.9999999999 (exactly 1 in FP32)
-  const R kb = R(3.0 * 0.3333333333);
-  const R c13 = kb * R(13.0 / 12.0), c14 = kb * R(0.25);
-  const R a1 = u3 - R(2) * u4 + u5, e1 = R(3) * u3 - R(4) * u4 + u5;
-  const R a2 = u2 - R(2) * u3 + u4, e2 = u2 - u4;
-  const R a3 = u1 - R(2) * u2 + u3, e3 = u1 - R(4) * u2 + R(3) * u3;
-  const R b1 = c13 * a1 * a1 + c14 * e1 * e1;
-  const R b2 = c13 * a2 * a2 + c14 * e2 * e2;
-  const R b3 = c13 * a3 * a3 + c14 * e3 * e3;
-  const R eps = R(1e-6);
-  const R q1 = b1 + eps, q2 = b2 + eps, q3 = b3 + eps;
-  const R w1 = R(0.3125) * wrcp(q1 * q1);
-  const R w2 = R(0.625) * wrcp(q2 * q2);
-  const R w3 = R(0.0625) * wrcp(q3 * q3);
-  const R tot = wrcp(w1 + w2 + w3);
-  return (w1 * tot) * (R(0.375) * u3 + R(0.75) * u4 - R(0.125) * u5) +
-         (w2 * tot) * (R(-0.125) * u2 + R(0.75) * u3 + R(0.375) * u4) +
-         (w3 * tot) * (R(0.375) * u1 - R(1.25) * u2 + R(1.875) * u3);
-}
-
-// FP32 form of the same value with fewer operations: the smoothness indicators
-// are taken times 12 (13 a^2 + 3 e^2, with eps times 12), which scales every
-// weight by 1/144 and cancels in the normalisation; the linear weights d_k are
-// folded into the candidate interpolants and into the weight sum, so that the
-// value is (sum_k r_k d_k p_k) / (sum_k d_k r_k) with r_k = 1 / q_k^2. Equal to
-// the form above up to rounding.
-template <>
-__device__ __forceinline__ float weno5<float>(float u1, float u2, float u3, float u4, float u5) {
-  const float a1 = u3 - 2.0f * u4 + u5, e1 = 3.0f * u3 - 4.0f * u4 + u5;
-  const float a2 = u2 - 2.0f * u3 + u4, e2 = u2 - u4;
-  const float a3 = u1 - 2.0f * u2 + u3, e3 = u1 - 4.0f * u2 + 3.0f * u3;
-  const float q1 = fmaf(13.0f * a1, a1, fmaf(3.0f * e1, e1, 12e-6f));
-  const float q2 = fmaf(13.0f * a2, a2, fmaf(3.0f * e2, e2, 12e-6f));
-  const float q3 = fmaf(13.0f * a3, a3, fmaf(3.0f * e3, e3, 12e-6f));
-  const float r1 = wrcp(q1 * q1), r2 = wrcp(q2 * q2), r3 = wrcp(q3 * q3);
-  const float sum = fmaf(0.3125f, r1, fmaf(0.625f, r2, 0.0625f * r3));
-  // d_k times the candidate interpolants (0.375 u3 + 0.75 u4 - 0.125 u5 etc.)
-  const float p1 = 0.1171875f * u3 + 0.234375f * u4 - 0.0390625f * u5;
-  const float p2 = -0.078125f * u2 + 0.46875f * u3 + 0.234375f * u4;
-  const float p3 = 0.0234375f * u1 - 0.078125f * u2 + 0.1171875f * u3;
-  return fmaf(r1, p1, fmaf(r2, p2, r3 * p3)) * wrcp(sum);
-}
+// WENO5-JS values at x_{i+1/2} (alternative_flux_FD.cpp:43-59), u1..u5 = u(i-2..i+2):
+// the smoothness indicators are written as the sums of squares they expand to,
+// e.g. (10 u3^2 - 31 u3 u4 + 25 u4^2 + 11 u3 u5 - 19 u4 u5 + 4 u5^2) / 3 =
+// 13/12 (u3 - 2 u4 + u5)^2 + 1/4 (3 u3 - 4 u4 + u5)^2; the weights are
+// d_k / (beta_k + 1e-6)^2 with d = (5/16, 10/16, 1/16), normalised. Below, the
+// indicators are taken times 12 (13 a^2 + 3 e^2, with eps times 12), which cancels
+// in the normalisation, and the linear weights d_k are folded into the candidate
+// interpolants and the weight sum.
 
 // FP32 WENO5 values of both sides of face q+1/2 from w(q-2 .. q+3):
-// um = weno5(w(q-2), .., w(q+2)) and up = weno5(w(q+3), .., w(q-1)), the same
-// smoothness indicators (times 12) and folded linear weights as weno5<float>.
+// um = weno5(w(q-2), .., w(q+2)) and up = weno5(w(q+3), .., w(q-1)).
 // The two sides share the second differences of the windows (q-1, q, q+1) and
 // (q, q+1, q+2) and two of their three candidate values (the parabola through
 // the same three cells at the same face): 4 second differences and 4
@@ -121,6 +72,35 @@ __device__ __forceinline__ void weno5_pair(float wm2, float wm1, float w0, float
   }
 }
 
+// The same in FP64, where a division is a dozen instructions and the range is wide:
+// the weights 1 / q_k^2 are taken times (q_1 q_2 q_3)^2, so that a side needs one
+// division instead of four. The reference scales the expanded indicators by the
+// literal 0.3333333333, i.e. the sums of squares by 0.9999999999: here eps by its
+// inverse. aw_faces at 150 x 140 x 90: 640 -> 399 us.
+__device__ __forceinline__ double weno5_side(double q1, double q2, double q3, double p1, double p2, double p3) {
+  const double a = q2 * q3, b = q1 * q3, c = q1 * q2;
+  const double a1 = a * a, a2 = b * b, a3 = c * c;
+  return fma(a1, p1, fma(a2, p2, a3 * p3)) / fma(0.3125, a1, fma(0.625, a2, 0.0625 * a3));
+}
+__device__ __forceinline__ void weno5_pair(double wm2, double wm1, double w0, double wp1, double wp2, double wp3,
+                                           double& um, double& up) {
+  constexpr double eps = 12e-6 / (3.0 * 0.3333333333);
+  const double Am2 = wm2 - 2.0 * wm1 + w0, Am1 = wm1 - 2.0 * w0 + wp1;
+  const double A0 = w0 - 2.0 * wp1 + wp2, A1 = wp1 - 2.0 * wp2 + wp3;
+  const double Cm2 = wm2 - w0, Cm1 = wm1 - wp1, C0 = w0 - wp2, C1 = wp1 - wp3;
+  const double Tm2 = fma(13.0 * Am2, Am2, eps), Tm1 = fma(13.0 * Am1, Am1, eps);
+  const double T0 = fma(13.0 * A0, A0, eps), T1 = fma(13.0 * A1, A1, eps);
+  const double e1 = fma(2.0, A0, C0), e3 = fma(2.0, Am2, -Cm2);
+  const double f1 = fma(2.0, Am1, -Cm1), f3 = fma(2.0, A1, C1);
+  // d1 times the two candidates shared by both sides, d3 times the extrapolations
+  const double PA = 0.1171875 * w0 + 0.234375 * wp1 - 0.0390625 * wp2;
+  const double PB = -0.0390625 * wm1 + 0.234375 * w0 + 0.1171875 * wp1;
+  const double Pm = 0.0234375 * wm2 - 0.078125 * wm1 + 0.1171875 * w0;
+  const double Pp = 0.0234375 * wp3 - 0.078125 * wp2 + 0.1171875 * wp1;
+  um = weno5_side(fma(3.0 * e1, e1, T0), fma(3.0 * Cm1, Cm1, Tm1), fma(3.0 * e3, e3, Tm2), PA, 2.0 * PB, Pm);
+  up = weno5_side(fma(3.0 * f1, f1, Tm1), fma(3.0 * C0, C0, T0), fma(3.0 * f3, f3, T1), PB, 2.0 * PA, Pp);
+}
+
 // Conservative elastic flux through a face of cofactor normal (n1, n2, n3)
 // (alternative_flux_FD.cpp:140-158).
 template <class R>
@@ -160,12 +140,7 @@ __device__ __forceinline__ void face_values(const StageArgs<R>& a, unsigned o, u
     const R* w = a.win + v * N;
     const R wm2 = *at(w, o - 2 * sb), wm1 = *at(w, o - sb), w0 = *at(w, o), wp1 = *at(w, o + sb),
             wp2 = *at(w, o + 2 * sb), wp3 = *at(w, o + 3 * sb);
-    if constexpr (sizeof(R) == 4) {
-      weno5_pair(wm2, wm1, w0, wp1, wp2, wp3, um[v], up[v]);
-    } else {
-      um[v] = weno5<R>(wm2, wm1, w0, wp1, wp2);
-      up[v] = weno5<R>(wp3, wp2, wp1, w0, wm1);
-    }
+    weno5_pair(wm2, wm1, w0, wp1, wp2, wp3, um[v], up[v]);
   }
   if constexpr (sizeof(R) == 4) {
     // the flux is linear in the state: F(u+) + F(u-) = F(u+ + u-), one flux
@@ -220,12 +195,14 @@ __global__ void __launch_bounds__(256) aw_faces(StageArgs<R> a) {
   if (i >= a.XE - H || j >= a.NY - 3) return;
   const unsigned o = (unsigned)i * (unsigned)sizeof(R) + (unsigned)j * a.rowb + (unsigned)k * a.planeb;
   const bool ji = j >= H, ki = k >= H;
-  if (ji && ki) {
+  // grid of three rows of blocks: a direction each
+  const int only = gridDim.y == 3 ? (int)blockIdx.y : -1;
+  if (ji && ki && only <= 0) {
     face_flux<R>(a, o, (unsigned)sizeof(R), 0);
     if (i == H) face_flux<R>(a, o - (unsigned)sizeof(R), (unsigned)sizeof(R), 0);
   }
-  if (ki) face_flux<R>(a, o, a.rowb, 1);
-  if (ji) face_flux<R>(a, o, a.planeb, 2);
+  if (ki && (only < 0 || only == 1)) face_flux<R>(a, o, a.rowb, 1);
+  if (ji && (only < 0 || only == 2)) face_flux<R>(a, o, a.planeb, 2);
 }
 
 template <class R>
@@ -663,7 +640,9 @@ __global__ void aw_record(const R* __restrict__ W, const R* __restrict__ cjm, lo
 template <class R>
 void launch_faces(const StageArgs<R>& a, hipStream_t st) {
   const long long nb = cg::interior_blocks(a.XE - 2 * H, a.NY - 5, a.NZ - 5, a.rtx, a.rty);
-  aw_faces<R><<<dim3((unsigned)nb), dim3(256), 0, st>>>(a);
+  // a few blocks, all resident at once: the three directions side by side instead of
+  // one after another in each thread (48 x 44 x 20: 158 -> 142 us per step)
+  aw_faces<R><<<dim3((unsigned)nb, nb <= 1024 ? 3 : 1), dim3(256), 0, st>>>(a);
 }
 
 template <class R>
