@@ -128,13 +128,6 @@ __device__ __forceinline__ void ld_face_coef(const float* cjm, long long N, unsi
 }
 static_assert(C_LAM == C_MU + 1 && C_B == C_MU + 2, "ld_face_coef reads mu, lambda, 1/rho in a row");
 
-// The corrected flux difference of a cell, f - d2/24 + 7 d4/5760 at its two
-// faces (update_cell), is linear in the face differences D(q) = F(q) - F(q-1):
-// DA D(c) + DB (D(c-1) + D(c+1)) + DG (D(c-2) + D(c+2)), whose weights add up to 1.
-constexpr float DA = float(1.0 + 30.0 / 288.0 + 42.0 / 5760.0);
-constexpr float DB = float(-16.0 / 288.0 - 28.0 / 5760.0);
-constexpr float DG = float(1.0 / 288.0 + 7.0 / 5760.0);
-
 // Values a wave keeps in LDS from step to step, one per lane and field, which
 // leaves the registers to the reconstruction (with them the xi/zeta kernel
 // spilled, and a spilled load is a load waited for): the differences of the last
@@ -156,8 +149,8 @@ __device__ __forceinline__ void add_face(Ring& r, int lane, bool complete, float
     const float fv = complete ? F[v] : 0.0f;
     const float D = fv - r.F[v][lane];
     r.F[v][lane] = fv;
-    F[v] = fmaf(DG, D + r.d[Q][v][lane],
-                fmaf(DB, r.d[(Q + 3) & 3][v][lane] + r.d[(Q + 1) & 3][v][lane], DA * r.d[(Q + 2) & 3][v][lane]));
+    F[v] = fmaf((float)DG, D + r.d[Q][v][lane],
+                fmaf((float)DB, r.d[(Q + 3) & 3][v][lane] + r.d[(Q + 1) & 3][v][lane], (float)DA * r.d[(Q + 2) & 3][v][lane]));
     r.d[Q][v][lane] = D;
     asm volatile("" ::"v"(F[v]));  // summed here, not where it is used with the four differences kept until then
   }
@@ -304,7 +297,7 @@ struct XZWave {
     for (int v = 0; v < 9; ++v) {
       const float f = xface ? F[v] : 0.0f;
       const float D = f - lane_prev(f), l = lane_prev(D), t = lane_next(D);
-      h[v] += hy[v] + fmaf(DA, D, fmaf(DB, l + t, DG * (lane_prev(l) + lane_next(t))));
+      h[v] += hy[v] + fmaf((float)DA, D, fmaf((float)DB, l + t, (float)DG * (lane_prev(l) + lane_next(t))));
     }
     if (own) {
 #pragma unroll
