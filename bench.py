@@ -52,10 +52,10 @@ def log(*a):
 
 def stage_bytes(coef_storage):
     """Algorithmic HBM bytes per cell per RK stage of the fused interior kernel:
-    stage 0 and 3 read W and write two arrays (3w + c), stages 1 and 2 read W, the
-    RK base and the accumulator and write two arrays (5w + c). Mean over stages."""
+    stage 0 reads and writes W (2w + c), stages 1 and 2 read the RK base too (3w + c),
+    stage 3 the base and the two earlier stage states (5w + c). Mean over stages."""
     c = C_BYTES[coef_storage]
-    return (2 * (3 * W_BYTES + c) + 2 * (5 * W_BYTES + c)) / 4.0
+    return (13 * W_BYTES + 4 * c) / 4.0
 
 
 def traffic_from_profiles(name):
@@ -72,12 +72,6 @@ def traffic_from_profiles(name):
         return None
 
 
-# ME-AWENO algorithmic bytes per cell and TVD stage (FP32): face kernel reads W
-# (36 B) and 12 coefficients (48 B) and writes 27 face fluxes (108 B); the update
-# reads the 27 fluxes, J, the stage input and the step-start state and writes
-# the stage output (108 + 4 + 3 * 36 B).
-AW_FACE_BYTES = 36 + 48 + 108
-AW_UPDATE_BYTES = 108 + 4 + 3 * 36
 # algorithmic bytes per cell and TVD-RK3 step of a fused ME-AWENO step: three
 # stages read the stage state (and the step-start state in stages 2 and 3) and
 # the 13 coefficients (9 cofactors, J, mu, lambda, 1/rho) and write the next
@@ -595,12 +589,10 @@ def bench_aweno(args):
     launch_ms = tm["interior_ms"] / max(tm["interior_n"], 1)
     upd_ms = tm["surface_ms"] / max(tm["surface_n"], 1)
     # algorithmic bytes of the fused minimum, 444 B per cell-step (8 w + 3 c'),
-    # over the measured step time; the face-flux buffer this build writes and
-    # re-reads is overhead, reported separately
+    # over the measured step time; the eta differences that the first kernel of a
+    # stage writes and the second reads are overhead, reported separately
     achieved = AW_ALG_BYTES * m.cells / (ms_step * 1e-3) / 1e9
-    NX, NY, NZ = m.shape_padded
-    face_cells = (NX - 5) * (NY - 5) * (NZ - 5)
-    flux_overhead = 2 * 27 * 4 * face_cells * 3  # 27 flux planes written and read per stage
+    eta_overhead = 2 * 9 * 4 * m.cells * 3  # nine planes written and read per stage
 
     l2 = None
     if not args.no_accuracy:
@@ -637,12 +629,12 @@ def bench_aweno(args):
         "l2_err_fp32_vs_fp64": l2,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": traffic_from_profiles("aw_faces_512x512x256_traffic.json"),
-                     "kernel": "aw_faces + aw_update (whole step)", "face_launch_ms": launch_ms,
+                     "traffic": traffic_from_profiles("aw_march_512x512x256_traffic.json"),
+                     "kernel": "aw_yflux + aw_xzstep (whole step)", "face_launch_ms": launch_ms,
                      "update_launch_ms": upd_ms, "alg_bytes_per_cell_step": AW_ALG_BYTES, "cells": m.cells,
-                     "flux_buffer_bytes_per_step": flux_overhead,
+                     "eta_difference_bytes_per_step": eta_overhead,
                      "note": "achieved = 444 B/cell-step (8 w + 3 c', fused minimum) x cells / step time; the "
-                             "27-plane face-flux buffer traffic is overhead outside the algorithmic bytes"},
+                             "eta differences between the two kernels of a stage are overhead outside them"},
         "cpu_baseline": cpu,
     }
     print(json.dumps(out), flush=True)
