@@ -199,10 +199,7 @@ template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
 __global__ __launch_bounds__(256) void cg_adj_a(AdjArgs<R> a, const TM* __restrict__ coef) {
   CellTile t;
   if (!interior_tile(blockIdx.x, a.nx, a.ny, a.nz, a.rtx, a.rty, t)) return;
-  const int i = H + t.i0 + (threadIdx.x & 63);
-  const int j = H + t.j0 + (threadIdx.x >> 6);
-  const int k = H + t.k;
-  if (i >= H + a.nx || j >= H + a.ny) return;
+  const int i = H + t.i, j = H + t.j, k = H + t.k;
   const long long p = (long long)i + (long long)a.NX * j + (long long)k * a.S;
   R gv[9];
 #pragma unroll
@@ -278,10 +275,7 @@ template <class R, int FB1, int FB2, int FB3, int STAGE>
 __global__ __launch_bounds__(256) void cg_adj_b(AdjArgs<R> a) {
   CellTile t;
   if (!interior_tile(blockIdx.x, a.nx, a.ny, a.nz, a.rtx, a.rty, t)) return;
-  const int i = H + t.i0 + (threadIdx.x & 63);
-  const int j = H + t.j0 + (threadIdx.x >> 6);
-  const int k = H + t.k;
-  if (i >= H + a.nx || j >= H + a.ny) return;
+  const int i = H + t.i, j = H + t.j, k = H + t.k;
   const long long p = (long long)i + (long long)a.NX * j + (long long)k * a.S;
   R gn[9];
   adj_b_cell<R, FB1, FB2, FB3, STAGE>(a, a.Z, k, p, gn);
@@ -302,10 +296,7 @@ __global__ __launch_bounds__(256) void cg_adj_ba(AdjArgs<R> a, const TM* __restr
   static_assert(STAGE >= 1 && STAGE <= 3, "pass A follows pass B of stages 3..1");
   CellTile t;
   if (!interior_tile(blockIdx.x, a.nx, a.ny, a.nz, a.rtx, a.rty, t)) return;
-  const int i = H + t.i0 + (threadIdx.x & 63);
-  const int j = H + t.j0 + (threadIdx.x >> 6);
-  const int k = H + t.k;
-  if (i >= H + a.nx || j >= H + a.ny) return;
+  const int i = H + t.i, j = H + t.j, k = H + t.k;
   const long long p = (long long)i + (long long)a.NX * j + (long long)k * a.S;
   R gn[9];
   adj_b_cell<R, FB1, FB2, FB3, STAGE>(a, a.Z, k, p, gn);

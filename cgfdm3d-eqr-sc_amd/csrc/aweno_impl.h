@@ -189,10 +189,7 @@ __global__ void __launch_bounds__(256) aw_faces(StageArgs<R> a) {
   // kernel.
   cg::CellTile t;
   if (!cg::interior_tile(blockIdx.x, a.XE - 2 * H, a.NY - 5, a.NZ - 5, a.rtx, a.rty, t)) return;
-  const int i = H + t.i0 + (threadIdx.x & 63);
-  const int j = 2 + t.j0 + (threadIdx.x >> 6);
-  const int k = 2 + t.k;
-  if (i >= a.XE - H || j >= a.NY - 3) return;
+  const int i = H + t.i, j = 2 + t.j, k = 2 + t.k;
   const unsigned o = (unsigned)i * (unsigned)sizeof(R) + (unsigned)j * a.rowb + (unsigned)k * a.planeb;
   const bool ji = j >= H, ki = k >= H;
   // grid of three rows of blocks: a direction each
@@ -292,10 +289,7 @@ template <class R>
 __device__ __forceinline__ void update_block(const StageArgs<R>& a, int block) {
   cg::CellTile t;
   if (!cg::interior_tile(block, a.XE - 2 * H, a.NY, a.NZ, a.rtx, a.rty, t)) return;
-  const int i = H + t.i0 + (threadIdx.x & 63);
-  const int j = t.j0 + (threadIdx.x >> 6);
-  const int k = t.k;
-  if (i >= a.XE - H || j >= a.NY) return;
+  const int i = H + t.i, j = t.j, k = t.k;
   update_cell<R>(a, i, j, k);
   if (i < 2 * H || i >= a.XE - 2 * H) {
     // ghost column: no right-hand side

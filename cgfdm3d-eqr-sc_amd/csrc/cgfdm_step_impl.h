@@ -365,10 +365,7 @@ template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
 __device__ __forceinline__ void cell_block(const StageArgs<R>& a, const TM* __restrict__ coef, int block) {
   CellTile t;
   if (!interior_tile(block, a.nx, a.ny, a.kend - a.kbeg, a.rtx, a.rty, t)) return;
-  const int i = H + t.i0 + (threadIdx.x & 63);
-  const int j = H + t.j0 + (threadIdx.x >> 6);
-  const int k = a.kbeg + t.k;
-  if (i >= H + a.nx || j >= H + a.ny) return;
+  const int i = H + t.i, j = H + t.j, k = a.kbeg + t.k;
   const long long N = a.N;
   const unsigned off = cell_off(a, i, j, k);
   const R* W = a.win;

@@ -102,17 +102,30 @@ __device__ __forceinline__ T* at(T* base, unsigned boff) {
 // each XCD gets an eighth: dealt whole they leave XCDs idle (333 x 150 x 117 has 19
 // regions: 35.3 -> 32.0 ms per 20 steps; the whole range cut into eighths costs the
 // shared edges: 512 x 512 x 256 140 -> 148 ms per 10). Returns false for padding blocks.
+//
+// A last tile column of at most 32 cells, in regions of whole rows, goes in blocks
+// of 32 columns by 8 rows: a wave takes two rows of it instead of one with half its
+// lanes idle (nx 150: 5 blocks where 6 were; 200: 7 for 8; 333: 11 for 12).
 struct CellTile {
-  int i0, j0, k;
+  int i, j, k;  // of the thread, from the first cell of the range
 };
 __device__ __host__ __forceinline__ int region_extent(int r, int n) { return (r <= 0 || r > n) ? n : r; }
+// blocks of a region's plane: whole tiles, and those of the narrow last column
+__device__ __host__ __forceinline__ void region_blocks(int nx, int ntx, int rtx, int rty, int& wide, int& narrow) {
+  const int r = nx % 64;
+  const bool has = rtx == ntx && r > 0 && r <= 32;
+  wide = (has ? rtx - 1 : rtx) * rty;
+  narrow = has ? (rty + 1) / 2 : 0;
+}
 
 __device__ __forceinline__ bool interior_tile(int b, int nx, int ny, int nk, int rtx, int rty, CellTile& t) {
   const int ntx = (nx + 63) / 64, nty = (ny + 3) / 4;
   rtx = region_extent(rtx, ntx);  // rtx <= 0: whole rows of tiles
   rty = region_extent(rty, nty);
   const int nrx = (ntx + rtx - 1) / rtx, nry = (nty + rty - 1) / rty;
-  const int per_plane = rtx * rty;
+  int wide, narrow;
+  region_blocks(nx, ntx, rtx, rty, wide, narrow);
+  const int per_plane = wide + narrow;
   const unsigned per_region = (unsigned)(per_plane * nk);  // the launch has fewer than 2^31 blocks
   const int nreg = nrx * nry;
   const unsigned xcd = (unsigned)b & 7u, seq = (unsigned)b >> 3, whole = (unsigned)(nreg / 8) * per_region;
@@ -126,23 +139,32 @@ __device__ __forceinline__ bool interior_tile(int b, int nx, int ny, int nk, int
     r = nreg / 8 * 8 + (int)(s / per_region);
     within = s % per_region;
   }
+  if (r >= nreg) return false;
   const int kk = (int)within / per_plane, q = (int)within - kk * per_plane;
-  const int ty = q / rtx, tx = q - ty * rtx;
   const int rx = r % nrx, ry = r / nrx;
-  const int txg = rx * rtx + tx, tyg = ry * rty + ty;
-  t.i0 = txg * 64;
-  t.j0 = tyg * 4;
+  int row;  // in the region
+  if (q < wide) {
+    const int w = narrow ? rtx - 1 : rtx, ty = q / w;
+    t.i = (rx * rtx + q - ty * w) * 64 + (int)(threadIdx.x & 63);
+    row = 4 * ty + (int)(threadIdx.x >> 6);
+  } else {
+    t.i = (ntx - 1) * 64 + (int)(threadIdx.x & 31);
+    row = 8 * (q - wide) + (int)(threadIdx.x >> 5);
+  }
+  t.j = 4 * rty * ry + row;
   t.k = kk;
-  return r < nreg && txg < ntx && tyg < nty;
+  return row < 4 * rty && t.i < nx && t.j < ny;
 }
 
 // number of blocks of the interior launch for interior_tile()
 inline long long interior_blocks(int nx, int ny, int nk, int rtx, int rty) {
-  const long long ntx = (nx + 63) / 64, nty = (ny + 3) / 4;
-  rtx = region_extent(rtx, (int)ntx);
-  rty = region_extent(rty, (int)nty);
-  const long long nregions = ((ntx + rtx - 1) / rtx) * ((nty + rty - 1) / rty);
-  const long long per_region = (long long)rtx * rty * nk;
+  const int ntx = (nx + 63) / 64, nty = (ny + 3) / 4;
+  rtx = region_extent(rtx, ntx);
+  rty = region_extent(rty, nty);
+  const long long nregions = (long long)((ntx + rtx - 1) / rtx) * ((nty + rty - 1) / rty);
+  int wide, narrow;
+  region_blocks(nx, ntx, rtx, rty, wide, narrow);
+  const long long per_region = (long long)(wide + narrow) * nk;
   return 8 * (nregions / 8 * per_region + (nregions % 8 * per_region + 7) / 8);
 }
 

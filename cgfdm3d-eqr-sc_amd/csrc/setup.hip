@@ -503,34 +503,34 @@ template void launch_pack_cmm<double>(const double*, const float*, double*, int,
 // grid took 0.9 s. Packed here and copied in one piece per 32 MB a plane takes 28 us
 // and a field 0.74 ms, bound by the transfer to pageable host memory.
 template <class T, class X>
-__global__ void __launch_bounds__(256) k_gather(const T* __restrict__ src, long long sa, long long sb, int na,
-                                                long long n, X* __restrict__ out, double sc) {
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(256) k_gather(const T* __restrict__ src, long long sa, long long sb,
+                                                unsigned na, unsigned n, X* __restrict__ out, double sc) {
+  const unsigned q = blockIdx.x * 256u + threadIdx.x;
   if (q >= n) return;
-  const long long b = q / na;
-  const T v = src[b * sb + (q - b * na) * sa];
+  const unsigned b = q / na;
+  const T v = src[(long long)b * sb + (long long)(q - b * na) * sa];
   if constexpr (std::is_integral<T>::value) out[q] = v;
   else out[q] = X((double)v * sc);
 }
 template <class T>
-__global__ void __launch_bounds__(256) k_scatter(T* __restrict__ dst, long long sb, int na, long long n,
+__global__ void __launch_bounds__(256) k_scatter(T* __restrict__ dst, long long sb, unsigned na, unsigned n,
                                                  const double* __restrict__ in, double sc) {
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+  const unsigned q = blockIdx.x * 256u + threadIdx.x;
   if (q >= n) return;
-  const long long b = q / na;
-  dst[b * sb + (q - b * na)] = T(in[q] * sc);
+  const unsigned b = q / na;
+  dst[(long long)b * sb + (q - b * na)] = T(in[q] * sc);
 }
 
 template <class T, class X>
 void launch_gather(const T* src, long long sa, long long sb, int na, long long rows, X* out, double sc,
                    hipStream_t st) {
-  const long long n = rows * na;
-  k_gather<T, X><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(src, sa, sb, na, n, out, sc);
+  const unsigned n = (unsigned)(rows * na);  // at most 16 M: one piece of the staging buffer
+  k_gather<T, X><<<(n + 255) / 256, 256, 0, st>>>(src, sa, sb, (unsigned)na, n, out, sc);
 }
 template <class T>
 void launch_scatter(T* dst, long long sb, int na, long long rows, const double* in, double sc, hipStream_t st) {
-  const long long n = rows * na;
-  k_scatter<T><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(dst, sb, na, n, in, sc);
+  const unsigned n = (unsigned)(rows * na);
+  k_scatter<T><<<(n + 255) / 256, 256, 0, st>>>(dst, sb, (unsigned)na, n, in, sc);
 }
 // integers: elements of 2, 4 or 8 bytes moved as they are
 template void launch_gather<unsigned short, unsigned short>(const unsigned short*, long long, long long, int,
