@@ -488,7 +488,8 @@ class Kernel:
             w.sset(o[0], 1, g(o[1], 1))
         elif op == "s_mov_b64":
             w.sset(o[0], 2, g(o[1], 2))
-        elif op in ("s_and_b64", "s_or_b64", "s_andn2_b64", "s_orn2_b64", "s_and_b32", "s_or_b32"):
+        elif op in ("s_and_b64", "s_or_b64", "s_andn2_b64", "s_orn2_b64", "s_and_b32", "s_or_b32",
+                    "s_andn2_b32"):
             wd = 2 if op.endswith("64") else 1
             a, b = g(o[1], wd), g(o[2], wd)
             mask = M64 if wd == 2 else M32
