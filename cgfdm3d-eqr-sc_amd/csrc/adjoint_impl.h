@@ -223,42 +223,28 @@ __device__ __forceinline__ void adj_b_cell(const AdjArgs<R>& a, const R* __restr
   // the surface pass scatters into layers ktop - 5 .. ktop only (7-point image
   // window of the three surface rows): the accumulator is read and cleared there
   const bool in_ls = a.fs && k >= H + a.nz - 6;
-  // the gathers axis by axis, the loads of an axis together (256 x 256 x 128, one
-  // gradient of 16 steps: 181 -> 171 ms; with all of a field's loads in turn the
-  // kernel held 210 registers), the loads of the read-modify-writes with the last
-  // axis: every load comes before the first store (the buffers are not known not to
-  // alias)
+  // gathers of all nine fields first, then the read-modify-writes: every load
+  // comes before the first store (the buffers are not known not to alias).
+  // Issuing an axis' 45 loads together, as the forward stages do, gains nothing
+  // here: at 256 x 256 x 128 cg_adj_ba takes 1.399 ms so and 1.394 grouped,
+  // cg_adj_b 0.416 and 0.419 (its stage 3 loses the third wave per SIMD).
   R l[9], ls[9], mv[9], ov[9];
 #pragma unroll
-  for (int ax = 0; ax < 3; ++ax) {
-    R f[9][5];
-    const long long d = FBv[ax] * sv[ax];
+  for (int v = 0; v < 9; ++v) {
+    l[v] = R(0);
 #pragma unroll
-    for (int v = 0; v < 9; ++v)
-#pragma unroll
-      for (int m = 0; m < 5; ++m) f[v][m] = Zin[(long long)(9 * ax + v) * N + p - (m - 1) * d];
-    if (ax == 2) {
-#pragma unroll
-      for (int v = 0; v < 9; ++v) {
-        const long long q = (long long)v * N + p;
-        ls[v] = R(0);
-        if constexpr (STAGE == 3 || STAGE > 0) mv[v] = a.mu[q];
-        if constexpr (STAGE != 3) ov[v] = a.out[q];
-      }
-      if (in_ls) {
-#pragma unroll
-        for (int v = 0; v < 9; ++v) ls[v] = a.Ls[(long long)v * N + p];
-      }
-    }
-    loads_issued();
-#pragma unroll
-    for (int v = 0; v < 9; ++v) {
+    for (int ax = 0; ax < 3; ++ax) {
+      const R* z = Zin + (long long)(9 * ax + v) * N + p;
+      const long long d = FBv[ax] * sv[ax];
       R acc = R(0);
 #pragma unroll
-      for (int m = 0; m < 5; ++m) acc += cw[m] * f[v][m];
-      acc = R(FBv[ax]) * acc * a.rDH;
-      l[v] = ax == 0 ? acc : l[v] + acc;
+      for (int m = 0; m < 5; ++m) acc += cw[m] * z[-(m - 1) * d];
+      l[v] += R(FBv[ax]) * acc * a.rDH;
     }
+    const long long q = (long long)v * N + p;
+    ls[v] = in_ls ? a.Ls[q] : R(0);
+    if constexpr (STAGE == 3 || STAGE > 0) mv[v] = a.mu[q];
+    if constexpr (STAGE != 3) ov[v] = a.out[q];
   }
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
