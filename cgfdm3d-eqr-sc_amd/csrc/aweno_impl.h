@@ -76,7 +76,9 @@ __device__ __forceinline__ void weno5_pair(float wm2, float wm1, float w0, float
 // the weights 1 / q_k^2 are taken times (q_1 q_2 q_3)^2, so that a side needs one
 // division instead of four. The reference scales the expanded indicators by the
 // literal 0.3333333333, i.e. the sums of squares by 0.9999999999: here eps by its
-// inverse. aw_faces at 150 x 140 x 90: 640 -> 399 us.
+// inverse. aw_faces at 150 x 140 x 90: 640 -> 399 us. These products are of the
+// eighth power of the state's differences and overflow from about 1e36 on, where
+// the squares alone reach 1e76: see weno5_wide.
 __device__ __forceinline__ double weno5_side(double q1, double q2, double q3, double p1, double p2, double p3) {
   const double a = q2 * q3, b = q1 * q3, c = q1 * q2;
   const double a1 = a * a, a2 = b * b, a3 = c * c;
@@ -99,6 +101,20 @@ __device__ __forceinline__ void weno5_pair(double wm2, double wm1, double w0, do
   const double Pp = 0.0234375 * wp3 - 0.078125 * wp2 + 0.1171875 * wp1;
   um = weno5_side(fma(3.0 * e1, e1, T0), fma(3.0 * Cm1, Cm1, Tm1), fma(3.0 * e3, e3, Tm2), PA, 2.0 * PB, Pm);
   up = weno5_side(fma(3.0 * f1, f1, Tm1), fma(3.0 * C0, C0, T0), fma(3.0 * f3, f3, T1), PB, 2.0 * PA, Pp);
+}
+
+// One side with the weights as they are defined, for faces whose values from
+// weno5_pair are not finite.
+__device__ __forceinline__ double weno5_wide(double u1, double u2, double u3, double u4, double u5) {
+  constexpr double eps = 12e-6 / (3.0 * 0.3333333333);
+  const double a1 = u3 - 2.0 * u4 + u5, e1 = 3.0 * u3 - 4.0 * u4 + u5;
+  const double a2 = u2 - 2.0 * u3 + u4, e2 = u2 - u4;
+  const double a3 = u1 - 2.0 * u2 + u3, e3 = u1 - 4.0 * u2 + 3.0 * u3;
+  const double q1 = fma(13.0 * a1, a1, fma(3.0 * e1, e1, eps)), q2 = fma(13.0 * a2, a2, fma(3.0 * e2, e2, eps)),
+               q3 = fma(13.0 * a3, a3, fma(3.0 * e3, e3, eps));
+  const double w1 = 0.3125 / (q1 * q1), w2 = 0.625 / (q2 * q2), w3 = 0.0625 / (q3 * q3), tot = w1 + w2 + w3;
+  return (w1 / tot) * (0.375 * u3 + 0.75 * u4 - 0.125 * u5) + (w2 / tot) * (-0.125 * u2 + 0.75 * u3 + 0.375 * u4) +
+         (w3 / tot) * (0.375 * u1 - 1.25 * u2 + 1.875 * u3);
 }
 
 // Conservative elastic flux through a face of cofactor normal (n1, n2, n3)
@@ -152,11 +168,34 @@ __device__ __forceinline__ void face_values(const StageArgs<R>& a, unsigned o, u
 #pragma unroll
     for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (F[v] - a.alpha * (up[v] - um[v]));
   } else {
-    R fm[9], fp[9];
-    phys_flux<R>(um, n1, n2, n3, mu, lam, b, fm);
-    phys_flux<R>(up, n1, n2, n3, mu, lam, b, fp);
+    auto flux = [&](R n1, R n2, R n3, R mu, R lam, R b) {
+      R fm[9], fp[9];
+      phys_flux<R>(um, n1, n2, n3, mu, lam, b, fm);
+      phys_flux<R>(up, n1, n2, n3, mu, lam, b, fp);
 #pragma unroll
-    for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (fp[v] + fm[v] - a.alpha * (up[v] - um[v]));
+      for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (fp[v] + fm[v] - a.alpha * (up[v] - um[v]));
+    };
+    flux(n1, n2, n3, mu, lam, b);
+    // an overflow in weno5_side makes one of its three weights infinite, so its
+    // numerator infinite or NaN, and its value and the flux not finite: one test per
+    // face (a step at 150 x 140 x 90 takes 2.056 ms without it and 2.058 with it)
+    R s = R(0);
+#pragma unroll
+    for (int v = 0; v < 9; ++v) s += F[v];
+    if (!(fabs(s) < __builtin_huge_val())) {
+      unsigned q = o;
+      asm("" : "+v"(q));  // loaded again: kept from above the nine fields would take 108 registers
+#pragma unroll
+      for (int v = 0; v < 9; ++v) {
+        auto w = [&](unsigned off) { return *at(a.win + v * N, off); };
+        um[v] = weno5_wide(w(q - 2 * sb), w(q - sb), w(q), w(q + sb), w(q + 2 * sb));
+        __builtin_amdgcn_sched_barrier(0);  // one side after the other: all at once would take 256 registers
+        up[v] = weno5_wide(w(q + 3 * sb), w(q + 2 * sb), w(q + sb), w(q), w(q - sb));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      flux(pl(a.cjm, N, 3 * d + 0, q), pl(a.cjm, N, 3 * d + 1, q), pl(a.cjm, N, 3 * d + 2, q), pl(a.cjm, N, C_MU, q),
+           pl(a.cjm, N, C_LAM, q), pl(a.cjm, N, C_B, q));
+    }
   }
 }
 

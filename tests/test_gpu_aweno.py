@@ -117,3 +117,27 @@ def test_aweno_marching_kernels_match_the_flux_array(solver_mod, monkeypatch, nx
         out.append(g.wavefield())
     for v in range(9):
         assert rel_l2(out[1][v], out[0][v]) < 1e-5, (v, rel_l2(out[1][v], out[0][v]))
+
+
+# The FP64 reconstruction over the range of the oracle's weights, which square the smoothness indicators: states
+# of 1e-30 (all weights from epsilon), 1 and 1e70. Ghost cells stay zero; FP64 tolerance as above.
+@pytest.mark.parametrize("scale", [1e-30, 1.0, 1e70])
+def test_aweno_fp64_range_of_the_state(scale, oracle_mod, solver_mod):
+    m = M.small_config(nx=22, ny=18, nz=14, npml=0, hills=2, layered=True, free_surface=True, nt=8)
+    m.stations, m.src_cells, m.src_rate = m.stations[:1], None, None
+    rng = np.random.default_rng(11)
+    init = [np.zeros((14 + 2 * H, 18 + 2 * H, 22 + 2 * H)) for _ in range(9)]
+    for v in range(9):
+        init[v][H:-H, H:-H, H:-H] = rng.standard_normal((14, 18, 22)) * (1.0 if v < 3 else 1e-7) * scale
+    print(f"state of {scale:g}, FP64, 3 steps", flush=True)
+    g = solver_mod.Solver(m, precision=8, scheme=solver_mod.SCHEME_AWENO)
+    o = oracle_mod.AwenoOracle(m, prec=8, threads=8)
+    for v in range(9):
+        g.set_field(v, init[v])
+        o.set_field(v, init[v])
+    g.step(3)
+    o.step(3)
+    for v in range(9):
+        a, b = g.field(v) / scale, o.field(v) / scale
+        assert np.isfinite(b).all() and np.linalg.norm(b) > 0
+        assert rel_l2(a, b) < 1e-10, (scale, v, rel_l2(a, b))
