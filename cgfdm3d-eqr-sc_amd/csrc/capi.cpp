@@ -600,11 +600,11 @@ struct Solver : SolverBase {
                           (long long)d.nx * d.ny * d.npml, (long long)d.npml * d.ny * d.nz,
                           (long long)d.nx * d.npml * d.nz, (long long)d.nx * d.ny * d.npml};
       for (int f = 0; f < 6; ++f) {
-        pml.f[f] = cg::FaceBuf<R>{nullptr, nullptr, nullptr, nullptr, 0};
+        pml.f[f] = cg::FaceBuf<R>{nullptr, nullptr, nullptr, 0};
         if (d.npml <= 0 || (f == 5 && !pml.has_z2)) continue;
         R* base = nullptr;
-        if ((rc = dalloc(&base, 36 * cnt[f]))) return rc;
-        pml.f[f] = cg::FaceBuf<R>{base, base + 9 * cnt[f], base + 18 * cnt[f], base + 27 * cnt[f], cnt[f]};
+        if ((rc = dalloc(&base, 27 * cnt[f]))) return rc;
+        pml.f[f] = cg::FaceBuf<R>{base, base + 9 * cnt[f], base + 18 * cnt[f], cnt[f]};
       }
     }
     // --- wavefield buffers and observers

@@ -69,9 +69,18 @@ __device__ __forceinline__ void stress_rows(const R* V, R m1, R m2, R m3, R mu, 
 // differences are exact or nearly so: one rounding of the result and the
 // roundings of x1..x3 weighted 1/3, 2/3, 1/3, against four roundings of an
 // accumulator.
+// rk_sum12: the part of the first two stages, which pml_face forms in stage 1.
+template <class R>
+__device__ __forceinline__ R rk_sum12(R a, R x1, R x2) {
+  return R(RK_B1 / RK_A2) * (x1 - a) + R(RK_B2 / RK_A3) * (x2 - a);
+}
+template <class R>
+__device__ __forceinline__ R rk_close(R a, R sum12, R x3, R h3) {
+  return a + (sum12 + R(RK_B3) * (x3 - a) + R(RK_B4) * h3);
+}
 template <class R>
 __device__ __forceinline__ R rk_close(R a, R x1, R x2, R x3, R h3) {
-  return a + (R(RK_B1 / RK_A2) * (x1 - a) + R(RK_B2 / RK_A3) * (x2 - a) + R(RK_B3) * (x3 - a) + R(RK_B4) * h3);
+  return rk_close(a, rk_sum12(a, x1, x2), x3, h3);
 }
 
 // 5-point MacCormack difference (without 1/DH) of f around f[0] with stride s.
@@ -100,22 +109,23 @@ __device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, con
   // extra: surface stress term added to hA[3..8] on the top layer.
   // Loads before stores: the buffers are not known not to alias, so a store between
   // two loads would make the compiler wait for each load in turn. All nine fields
-  // together (five and four in the last stage, which reads four buffers): the
+  // together (five and four in the last stage, which reads three buffers): the
   // stencil's registers are free at this point.
+  // An auxiliary state is read and written by its own cell only, so two buffers hold
+  // the stage states: stage 1 has both X1 and X2 at hand and leaves their part of the
+  // closing sum in place of X1, stage 2 writes X3 in place of X2. 2 + 4 + 3 + 4 = 13
+  // transfers per step, as many as with a buffer for each state.
   constexpr int G = STAGE == 3 ? 5 : 9;
 #pragma unroll
   for (int g = 0; g < 9; g += G) {
-    R cur[G], av[G], x1[G], x2[G];
+    R cur[G], av[G], s12[G];
 #pragma unroll
     for (int u = 0; u < G; ++u) {
       if (g + u >= 9) break;
       const long long q = (long long)(g + u) * F.cnt + pos;
-      cur[u] = (STAGE == 0 ? F.a : STAGE == 1 ? F.x1 : STAGE == 2 ? F.x2 : F.x3)[q];
+      cur[u] = (STAGE == 0 ? F.a : STAGE == 1 ? F.x1 : F.x2)[q];
       if constexpr (STAGE != 0) av[u] = F.a[q];
-      if constexpr (STAGE == 3) {
-        x1[u] = F.x1[q];
-        x2[u] = F.x2[q];
-      }
+      if constexpr (STAGE == 3) s12[u] = F.x1[q];
     }
     loads_issued();
     const R ad = d + al;
@@ -128,9 +138,12 @@ __device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, con
       if (has_extra && v >= 3) hA += extra[v - 3] * DT;
       h[v] -= be * cur[u] * DT;
       if constexpr (STAGE == 0) F.x1[q] = cur[u] + R(RK_A2) * hA;
-      else if constexpr (STAGE == 1) F.x2[q] = av[u] + R(RK_A3) * hA;
-      else if constexpr (STAGE == 2) F.x3[q] = av[u] + hA;
-      else F.a[q] = rk_close(av[u], x1[u], x2[u], cur[u], hA);
+      else if constexpr (STAGE == 1) {
+        const R x2 = av[u] + R(RK_A3) * hA;
+        F.x1[q] = rk_sum12(av[u], cur[u], x2);
+        F.x2[q] = x2;
+      } else if constexpr (STAGE == 2) F.x2[q] = av[u] + hA;
+      else F.a[q] = rk_close(av[u], s12[u], cur[u], hA);
     }
   }
 }

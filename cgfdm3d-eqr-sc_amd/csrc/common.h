@@ -53,15 +53,14 @@ template <> struct Bits16<__hip_bfloat16> {
 // the default keeps the reference meaning (xi_x ... zt_z in 1/m).
 enum { M_XIX = 0, M_XIY, M_XIZ, M_ETX, M_ETY, M_ETZ, M_ZTX, M_ZTY, M_ZTZ, M_MU, M_LAM, M_B, M_NCOEF };
 
-// One PML face slab (reference pml_deriv.cpp:17-37): four RK buffers of 9 SoA
+// One PML face slab (reference pml_deriv.cpp:17-37): three RK buffers of 9 SoA
 // components over `cnt` cells. a = state at the step start (and the final
-// state), x1..x3 = the stage states, as the wavefield's A, B, C, D.
+// state); x1, x2 = the stage states, each in place of an earlier one (pml_face).
 template <class R>
 struct FaceBuf {
   R* a;
   R* x1;
   R* x2;
-  R* x3;
   long long cnt;
 };
 
