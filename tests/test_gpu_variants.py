@@ -71,3 +71,43 @@ def test_stage_launches_match_oracle(nx, ny, nz, coef, oracle_mod):
     for v in range(9):
         err = rel_l2(g.field(v), o.field(v))
         assert err < tol, (nx, ny, nz, coef, v, err)
+
+
+# The block order from a state that fills the grid, so that a cell left out, done twice or misplaced shows: last
+# tile columns of 1, 32 (in blocks of 32 by 8), 33 and 63 cells, 5 to 33 tile rows in regions of 1, 2 (the default)
+# and 3, region counts that eight divides and does not, regions of one tile column; one launch per stage (up to
+# 1024 blocks) and two. Tolerances as above.
+@pytest.mark.parametrize("nx,ny,nz,fs,prec,coef,env", [
+    (65, 18, 12, True, 4, 0, {}),
+    (96, 22, 13, False, 4, 0, {}),
+    (97, 33, 12, True, 8, 0, {"CGFDM_INTERIOR_RTY": "3"}),
+    (127, 64, 11, False, 8, 0, {"CGFDM_INTERIOR_RTY": "1"}),
+    (31, 130, 14, True, 4, 1, {}),
+    (130, 100, 26, True, 4, 0, {}),
+    (150, 66, 24, True, 4, 2, {"CGFDM_INTERIOR_RTY": "3"}),
+    (140, 40, 30, True, 4, 0, {"CGFDM_INTERIOR_RTX": "1"}),
+])
+def test_block_order_reaches_every_cell(nx, ny, nz, fs, prec, coef, env, oracle_mod, monkeypatch):
+    from cgfdm_amd import model as M
+    from cgfdm_amd import solver
+    H = M.HALO
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    m = M.small_config(nx=nx, ny=ny, nz=nz, npml=4, hills=2, layered=True, free_surface=fs, nt=8)
+    print(f"{nx}x{ny}x{nz} fs {fs} precision {prec} coef {coef} {env}, 3 steps", flush=True)
+    g = solver.Solver(m, precision=prec, coef_storage=coef)
+    o = oracle_mod.Oracle(m, prec=prec if coef == 0 else 8, threads=8)
+    rng = np.random.default_rng(nx)
+    for v in range(9):
+        w = np.zeros(g.shape)
+        w[H:-H, H:-H, H:-H] = rng.standard_normal((nz, ny, nx)) * (1.0 if v < 3 else 1e7)
+        g.set_field(v, w)
+        o.set_field(v, w)
+    g.step(3)
+    o.step(3)
+    tol = 1e-10 if prec == 8 else 3e-5 if coef == 0 else 5e-3 if coef == 1 else 4e-2
+    for v in range(9):
+        a, b = g.field(v), o.field(v)
+        assert rel_l2(a, b) < tol, (v, rel_l2(a, b))
+        # the last 32 columns by themselves
+        assert rel_l2(a[..., -H - 32:], b[..., -H - 32:]) < tol, v
