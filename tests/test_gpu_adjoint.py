@@ -267,3 +267,32 @@ def test_adjoint_with_recomputed_stages_matches_oracle(oracle_mod, solver_mod, m
     for k in ("gmu", "glam", "gb", "grate"):
         scale = np.abs(r[k]).max()
         np.testing.assert_allclose(gr[k], r[k], rtol=0, atol=1e-10 * scale, err_msg=k)
+
+
+@pytest.mark.parametrize("nx,ny,env", [(70, 21, {}), (100, 17, {"CGFDM_ADJOINT_PIPE": "0"}), (128, 13, {})])
+def test_adjoint_with_several_tile_columns_matches_oracle(nx, ny, env, oracle_mod, solver_mod, monkeypatch):
+    """Whole 64-column tiles beside a last column of 6 cells (blocks of 32 by 8) or of 36, and whole tiles only:
+    stations all over the grid and a state that fills it, so that every cell has a gradient."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    nst, ck, H = 4, 2, M.HALO
+    m = M.small_config(nx=nx, ny=ny, nz=12, npml=3, hills=2, free_surface=True, nt=nst)
+    rng = np.random.default_rng(nx)
+    m.stations = np.ascontiguousarray(np.stack([rng.integers(0, n, 300) + H for n in (nx, ny, 12)], 1), np.int32)
+    print(f"adjoint {nx}x{ny}x12 {env}, {nst} steps, 300 stations", flush=True)
+    g = solver_mod.Solver(m, precision=8)
+    o = oracle_mod.Oracle(m, prec=8, threads=8)
+    for v in range(9):
+        w = np.zeros(g.shape)
+        w[H:-H, H:-H, H:-H] = rng.standard_normal((12, ny, nx)) * (1.0 if v < 3 else 1e7)
+        g.set_field(v, w)
+        o.set_field(v, w)
+    gr = g.adjoint(g.forward_record(nst, ck))
+    r = oracle_mod.adjoint_misfit(o, nst, np.zeros((300, nst, 3)), npts=len(m.src_cells), nt_src=m.src_rate.shape[1])
+    for k in ("gmu", "glam", "gb"):
+        inner = r[k][H:-H, H:-H, H:-H]
+        assert (np.abs(inner) > 1e-6 * np.abs(inner).max()).mean() > 0.5, k
+    for k in ("gmu", "glam", "gb", "grate"):
+        scale = np.abs(r[k]).max()
+        assert scale > 0, k
+        np.testing.assert_allclose(gr[k], r[k], rtol=0, atol=1e-10 * scale, err_msg=k)
