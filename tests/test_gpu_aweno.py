@@ -141,3 +141,19 @@ def test_aweno_fp64_range_of_the_state(scale, oracle_mod, solver_mod):
         a, b = g.field(v) / scale, o.field(v) / scale
         assert np.isfinite(b).all() and np.linalg.norm(b) > 0
         assert rel_l2(a, b) < 1e-10, (scale, v, rel_l2(a, b))
+
+
+# The marching kernels, which large grids take, on the oracle cases of this file: fields within the FP32 tolerance
+# above, station records and PGV within that of the seismograms.
+@pytest.mark.parametrize("name", list(CASES))
+def test_aweno_marching_kernels_match_oracle(name, oracle_mod, solver_mod, monkeypatch):
+    monkeypatch.setenv("CGFDM_AWENO_MARCH", "1")
+    m, g, o = run_pair(name, oracle_mod, solver_mod, 4, 12)
+    assert g.kernel_name(0) == "aw_yflux"
+    for v in range(9):
+        assert rel_l2(g.field(v), o.field(v)) < 1e-5, (name, v, rel_l2(g.field(v), o.field(v)))
+    sg, so = g.stations(), o.stations()
+    assert rel_l2(sg[..., :3], so[..., :3]) < 1e-4 and rel_l2(sg[..., 3:], so[..., 3:]) < 1e-4
+    if m.free_surface:
+        assert rel_l2(g.pgv(), o.pgv()) < 1e-4
+        assert rel_l2(g.surface_displacement(), o.surface_dis()) < 1e-4
