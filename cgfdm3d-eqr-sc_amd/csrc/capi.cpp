@@ -105,18 +105,37 @@ struct SolverBase {
 
   // Staging buffer of the getters and setters, part of the solver: rows are packed
   // into it on the device (launch_gather) and copied in one piece, STAGE bytes at a
-  // time; a row always fits.
+  // time. It takes what the solver leaves free, down to one row, and gives way to
+  // later allocations (dalloc): no grid is refused for it.
   static constexpr long long STAGE = 32LL << 20;
   double* stage = nullptr;
   long long stage_n = 0;  // doubles
+  long long stage_row() const { return std::max(pXe, std::max(pNY, pNZ)); }
   int alloc_stage() {
-    const long long tN = (long long)pXe * pNY * pNZ;
-    stage_n = std::max(std::min(tN, STAGE / 8), (long long)std::max(pXe, std::max(pNY, pNZ)));
-    return dalloc(&stage, stage_n);
+    const long long row = stage_row();
+    stage = nullptr;
+    for (stage_n = std::max(std::min((long long)pXe * pNY * pNZ, STAGE / 8), row);; stage_n = std::max(stage_n / 2, row)) {
+      const int rc = dalloc(&stage, stage_n);
+      if (rc != CGFDM_ERR_ALLOC || stage_n == row) return rc;
+    }
+  }
+  // makes room: hipMalloc of nb bytes with the staging buffer out of the way, which
+  // is then allocated again in what is left (a row of it is held back meanwhile)
+  hipError_t malloc_for_stage(void** q, size_t nb) {
+    if (!stage || stage_n <= stage_row()) return hipErrorOutOfMemory;
+    (void)hipStreamSynchronize(stream);  // nothing queued uses it; its copies are waited for by the calls that make them
+    dfree(stage);
+    void* row = nullptr;
+    (void)hipMalloc(&row, sizeof(double) * stage_row());
+    const hipError_t e = hipMalloc(q, nb);
+    (void)hipFree(row);
+    (void)alloc_stage();
+    return e;
   }
   // `rows` rows of `na` elements, sa apart, a row every sb elements, to host as X
   template <class T, class X>
   int gather(const T* src, long long sa, long long sb, int na, long long rows, X* host, double sc) {
+    if (!stage) return fail(CGFDM_ERR_ALLOC, "no staging buffer");
     const long long step = std::max(1LL, stage_n * 8 / (long long)sizeof(X) / na);
     for (long long r = 0; r < rows; r += step) {
       const long long m = std::min(step, rows - r);
@@ -180,6 +199,7 @@ struct SolverBase {
   }
   template <class T>
   int volume_in(T* dev, const double* host, double sc) {
+    if (!stage) return fail(CGFDM_ERR_ALLOC, "no staging buffer");
     const long long rows = (long long)pNY * pNZ, step = std::max(1LL, stage_n / pXe);
     for (long long r = 0; r < rows; r += step) {
       const long long m = std::min(step, rows - r);
@@ -208,15 +228,19 @@ struct SolverBase {
   double ranges[8] = {0};
   long long bytes = 0;
 
-  // device allocations owned by the solver, zero-filled, and their sizes
+  // device allocations owned by the solver, zero-filled, and their sizes. One that
+  // does not fit beside the staging buffer is tried again without it, unless it is
+  // `optional`.
   std::vector<void*> allocs;
   std::vector<size_t> alloc_bytes;
   template <class X>
-  int dalloc(X** p, long long count) {
+  int dalloc(X** p, long long count, bool optional = false) {
     size_t nb = (size_t)count * sizeof(X);
     if (nb == 0) nb = 16;
     void* q = nullptr;
     hipError_t e = hipMalloc(&q, nb);
+    if (e != hipSuccess) (void)hipGetLastError();  // reported by the status, not by a later launch check
+    if (e != hipSuccess && !optional) e = malloc_for_stage(&q, nb);
     if (e != hipSuccess) return fail(CGFDM_ERR_ALLOC, "hipMalloc of " + std::to_string(nb) + " bytes failed");
     e = hipMemsetAsync(q, 0, nb, stream);
     if (e != hipSuccess) {
@@ -521,7 +545,6 @@ struct Solver : SolverBase {
     pNY = NY;
     pNZ = NZ;
     pXe = tNX;
-    if ((rc = alloc_stage())) return rc;
     if constexpr (kPacked16) {
       unsigned* words = nullptr;
       if ((rc = galloc(&words, (long long)(cg::M_NCOEF / 2) * N))) return rc;
@@ -614,6 +637,7 @@ struct Solver : SolverBase {
     if ((rc = galloc(&D, 9 * N))) return rc;
     if ((rc = dalloc(&pgv, 2LL * d.nx * d.ny))) return rc;
     if ((rc = dalloc(&dis, 3 * S))) return rc;
+    if ((rc = alloc_stage())) return rc;
     HIPCHK(hipStreamSynchronize(stream));
     return CGFDM_OK;
   }
@@ -1002,7 +1026,7 @@ struct Solver : SolverBase {
       if (hipMemGetInfo(&fre, &tot) == hipSuccess) budget = 0.85 * ((double)fre - reserve);
       (void)hipGetLastError();
     }
-    if (need <= budget && dalloc(&adj_stages, 36LL * N * ck) != CGFDM_OK) {
+    if (need <= budget && dalloc(&adj_stages, 36LL * N * ck, true) != CGFDM_OK) {
       adj_stages = nullptr;
       (void)hipGetLastError();
     }
@@ -1387,7 +1411,6 @@ struct AwenoSolver : SolverBase {
     pNY = NY;
     pNZ = NZ;
     pXe = tNX;
-    if ((rc = alloc_stage())) return rc;
     if ((rc = galloc(&cjm, (long long)aw::C_N * N))) return rc;
     if ((rc = repack(cjm, cjm_t, (long long)aw::C_N * NY * NZ, true))) return rc;
     HIPCHK(hipStreamSynchronize(stream));
@@ -1399,6 +1422,7 @@ struct AwenoSolver : SolverBase {
     if (!march && (rc = galloc(&F, 27 * N))) return rc;
     if ((rc = dalloc(&pgv, 2LL * d.nx * d.ny))) return rc;
     if ((rc = dalloc(&dis, 3 * S))) return rc;
+    if ((rc = alloc_stage())) return rc;
     HIPCHK(hipStreamSynchronize(stream));
     return CGFDM_OK;
   }

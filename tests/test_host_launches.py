@@ -38,3 +38,46 @@ for npml in (0, 7):
 cells = 7 * (2 * 26 * 22 + 2 * 31 * 22 + {1 if free_surface else 2} * 31 * 26)
 assert used[1] - used[0] == 27 * cells * {precision}, (used, cells)
 """)
+
+
+@pytest.mark.parametrize("scheme,precision", [("CGFDM", 4), ("CGFDM", 8), ("AWENO", 4), ("AWENO", 8)])
+def test_staging_buffer_gives_way_to_the_solver(scheme, precision):
+    """The buffer that fields and slices are packed into takes only memory that is left: a grid that fits without it
+    is made, station records that fit without it too, and fields and slices are still copied, row by row if need
+    be."""
+    run(f"""
+import numpy as np
+def make():
+    m = M.small_config(nx=40, ny=33, nz=30, npml=4, nt=4)
+    m.stations, m.src_cells, m.src_rate = None, None, None
+    return m, S.Solver(m, precision={precision}, scheme=S.SCHEME_{scheme})
+def copies(g):
+    for c in range(9):
+        g.set_field(c, np.zeros(g.shape))
+        assert g.field(c).shape == g.shape
+        assert g.slice(c, 0, 5).size == 33 * 30 and g.slice(c, 1, 5).size == 40 * 30 and g.slice(c, 2, 5).size == 40 * 33
+    g.step(1)
+    g.synchronize()
+def pieces(g):
+    sim.names()
+    g.field(3)
+    return sim.names().count('k_gather')
+m, g = make()
+full, stage = g.device_bytes(), 8 * g.N
+assert pieces(g) == 1
+g.close()
+assert sim.used == 0
+sim.limit = full - stage + 8 * 46  # the grid and one row of 46
+m, g = make()
+assert pieces(g) == 39 * 36
+copies(g)
+g.close()
+sim.limit = full + 4096
+m, g = make()
+assert pieces(g) == 1
+n = (4096 + stage // 2) // (4 * 9 * 4)
+S._check(g.L.cgfdm_set_stations(g.h, n, S._ptr(np.full((n, 3), 5, np.int32))))
+assert 1 < pieces(g) < 40 and g.device_bytes() == sim.used <= sim.limit
+copies(g)
+g.close()
+""")
