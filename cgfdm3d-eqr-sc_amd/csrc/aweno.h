@@ -29,6 +29,15 @@ template <class R>
 void launch_faces(const StageArgs<R>& a, hipStream_t st);
 template <class R>
 void launch_update(const StageArgs<R>& a, int nx, int ny, hipStream_t st);
+// Blocks of both updates where launch_update takes them in one launch (aw_update_both),
+// else 0. FP32, up to 1024 blocks; us per step in two launches and in one: 48 x 44 x 20
+// 108 and 85, 64 x 70 x 44 (about 1000) 173 and 145. FP64 would need 248 registers.
+template <class R>
+inline long long one_update_blocks(const StageArgs<R>& a, int nx, int ny) {
+  const long long nb = cg::interior_blocks(a.XE - 2 * cg::H, a.NY, a.NZ, a.rtx, a.rty) +
+                       3LL * ((nx + 63) / 64) * ((ny + 3) / 4);
+  return sizeof(R) == 4 && nb <= 1024 ? nb : 0;
+}
 // The stage in two marching kernels without the flux array (aweno_march.h): y
 // first, then x, z and the top layers.
 void launch_march_y(const StageArgs<float>& a, int nx, int ny, hipStream_t st);

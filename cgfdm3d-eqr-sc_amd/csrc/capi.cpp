@@ -750,8 +750,12 @@ struct Solver : SolverBase {
   int step(int n) override { return step_impl(n, true); }
 
   const char* kernel_name(int which) const override {
+    if (which != 0 && which != 1) return nullptr;
+    cg::StageArgs<R> a{};
+    a.nx = d.nx; a.ny = d.ny; a.nz = d.nz; a.kbeg = cg::H; a.kend = cg::H + d.nz - 3;
+    a.rty = rty; a.rtx = rtx; a.zreg = zreg; a.kc = kc;
+    if (d.free_surface && cg::one_launch_blocks(a)) return "cg_stage";
     if (which == 1) return "cg_surface";
-    if (which != 0) return nullptr;
     if (std::is_same<R, float>::value && std::is_same<TM, float>::value && kc < 0 && !galign) return "cg_pair";
     if (std::is_same<R, float>::value && kc == 1) return "cg_plane";
     if (std::is_same<R, float>::value && kc > 1) return "cg_zcol";
@@ -820,12 +824,13 @@ struct Solver : SolverBase {
         // the surface and the interior stage on one stream: they may run side by
         // side, but the events that fork and join a second stream cost more (us per
         // step: 24 x 20 x 16 146 -> 95, 128 x 128 x 64 321 -> 286, 512 x 512 x 256
-        // 14014 -> 14033). With timing on, each is launched and timed by itself.
+        // 14014 -> 14033). Timing times the same launches, one taken in one as the interior's.
         cg::SurfArgs<R> sa{jac, rdzdx, rdzdy, observe ? pgv : nullptr, dis};
         if (!timing_on) {
           if (int rc = launch_stage(a, sa, fb)) return rc;
         } else {
-          if (d.free_surface) {
+          const bool one = d.free_surface && cg::one_launch_blocks(a);
+          if (d.free_surface && !one) {
             const size_t fp = next_pair(1);
             HIPCHK(hipEventRecord(ev[fp].a, stream));
             LAUNCHCHK((cg::launch_surface<R, TM>(a, coef, sa, fb[0], fb[1], fb[2], stream)), "surface stage");
@@ -833,7 +838,11 @@ struct Solver : SolverBase {
           }
           const size_t ip = next_pair(0);
           HIPCHK(hipEventRecord(ev[ip].a, stream));
-          LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
+          if (one) {
+            if (int rc = launch_stage(a, sa, fb)) return rc;
+          } else {
+            LAUNCHCHK((cg::launch_interior<R, TM>(a, coef, fb[0], fb[1], fb[2], stream)), "interior stage");
+          }
           HIPCHK(hipEventRecord(ev[ip].b, stream));
         }
         fb[0] = -fb[0];
@@ -1490,7 +1499,12 @@ struct AwenoSolver : SolverBase {
   }
 
   const char* kernel_name(int which) const override {
-    return which == 0 ? (march ? "aw_yflux" : "aw_faces") : which == 1 ? (march ? "aw_xzstep" : "aw_update") : nullptr;
+    if (which != 0 && which != 1) return nullptr;
+    if (march) return which == 0 ? "aw_yflux" : "aw_xzstep";
+    if (which == 0) return "aw_faces";
+    aw::StageArgs<R> a{};
+    a.XE = tNX; a.NY = NY; a.NZ = NZ; a.rtx = rtx; a.rty = rty;
+    return aw::one_update_blocks(a, d.nx, d.ny) ? "aw_update_both" : "aw_update";
   }
 
   int step(int n) override {

@@ -50,6 +50,22 @@ template <class R, class TM>
 int launch_surface(StageArgs<R> a, const TM* coef, SurfArgs<R> s, int fb1, int fb2, int fb3, hipStream_t st);
 template <class R, class TM>
 int launch_stage(StageArgs<R> a, const TM* coef, SurfArgs<R> s, int fb1, int fb2, int fb3, hipStream_t st);
+// Interior and surface blocks of a stage under a free surface where launch_stage takes
+// them in one launch (cg_stage), else 0. FP32: up to 1024 blocks, twice what the 256
+// CUs hold at two blocks each (the registers of the surface part); the surface
+// first and the interior after it otherwise. us per step in two launches and in one:
+// 24 x 20 x 16 (80 blocks) 78 and 48, 64 x 60 x 40 (600) 113 and 87, 64 x 64 x 62 (992)
+// 128 and 99; above the line still 172 and 158 at 2000 blocks, with the gain falling.
+// FP64 would need more registers than there are for two blocks.
+template <class R>
+inline long long one_launch_blocks(const StageArgs<R>& a) {
+  const int nk = a.kend - a.kbeg;
+  if (sizeof(R) != 4 || a.kc != 0 || a.zreg != 0 || a.stage < 0 || a.stage > 3 || nk <= 0 || a.nx <= 0 || a.ny <= 0)
+    return 0;
+  const long long nb = 3LL * ((a.nx + 63) / 64) * ((a.ny + 3) / 4) +
+                       interior_blocks(a.nx, a.ny, nk, a.rtx, a.rty < 1 ? 1 : a.rty);
+  return nb <= 1024 ? nb : 0;
+}
 template <class R>
 void launch_source(R* W, long long N, int np, const long long* cell, const R* rate, int srcIt, R tw, R DT, hipStream_t st);
 template <class R>

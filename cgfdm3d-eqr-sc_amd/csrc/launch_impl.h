@@ -193,32 +193,24 @@ int launch_surface(StageArgs<R> a, const TM* coef, SurfArgs<R> s, int fb1, int f
   return LAUNCH_OK;
 }
 
-// Interior and surface of a stage under a free surface. FP32: in one launch up to
-// 1024 blocks, twice what the 256 CUs hold at two blocks each (the registers of the
-// surface part), else the surface first and the interior after it. us per step: 24 x
-// 20 x 16 (80 blocks) 81 -> 49, a gradient of 64 x 60 x 40 (600 blocks, 24 steps)
-// 20.0 -> 18.3 ms. FP64 would need more registers than there are for two blocks.
+// Interior and surface of a stage under a free surface.
 template <class R, class TM>
 int launch_stage(StageArgs<R> a, const TM* coef, SurfArgs<R> s, int fb1, int fb2, int fb3, hipStream_t st) {
-  const int nk = a.kend - a.kbeg;
   if constexpr (std::is_same<R, float>::value) {
-    if (a.kc == 0 && a.zreg == 0 && a.stage >= 0 && a.stage <= 3 && nk > 0 && a.nx > 0 && a.ny > 0) {
+    if (const long long nb = one_launch_blocks(a)) {
       if (a.rty < 1) a.rty = 1;
-      const long long nb = 3LL * ((a.nx + 63) / 64) * ((a.ny + 3) / 4) + interior_blocks(a.nx, a.ny, nk, a.rtx, a.rty);
-      if (nb <= 1024) {
-        const dim3 grid((unsigned)nb), block(256);
-        switch (fb_index(fb1, fb2, fb3)) {
-          case 0: both_stage<R, TM, -1, -1, -1>(a, coef, s, grid, block, st); break;
-          case 1: both_stage<R, TM, 1, -1, -1>(a, coef, s, grid, block, st); break;
-          case 2: both_stage<R, TM, -1, 1, -1>(a, coef, s, grid, block, st); break;
-          case 3: both_stage<R, TM, 1, 1, -1>(a, coef, s, grid, block, st); break;
-          case 4: both_stage<R, TM, -1, -1, 1>(a, coef, s, grid, block, st); break;
-          case 5: both_stage<R, TM, 1, -1, 1>(a, coef, s, grid, block, st); break;
-          case 6: both_stage<R, TM, -1, 1, 1>(a, coef, s, grid, block, st); break;
-          default: both_stage<R, TM, 1, 1, 1>(a, coef, s, grid, block, st); break;
-        }
-        return LAUNCH_OK;
+      const dim3 grid((unsigned)nb), block(256);
+      switch (fb_index(fb1, fb2, fb3)) {
+        case 0: both_stage<R, TM, -1, -1, -1>(a, coef, s, grid, block, st); break;
+        case 1: both_stage<R, TM, 1, -1, -1>(a, coef, s, grid, block, st); break;
+        case 2: both_stage<R, TM, -1, 1, -1>(a, coef, s, grid, block, st); break;
+        case 3: both_stage<R, TM, 1, 1, -1>(a, coef, s, grid, block, st); break;
+        case 4: both_stage<R, TM, -1, -1, 1>(a, coef, s, grid, block, st); break;
+        case 5: both_stage<R, TM, 1, -1, 1>(a, coef, s, grid, block, st); break;
+        case 6: both_stage<R, TM, -1, 1, 1>(a, coef, s, grid, block, st); break;
+        default: both_stage<R, TM, 1, 1, 1>(a, coef, s, grid, block, st); break;
       }
+      return LAUNCH_OK;
     }
   }
   if (const int r = launch_surface<R, TM>(a, coef, s, fb1, fb2, fb3, st); r > LAUNCH_EMPTY) return r;

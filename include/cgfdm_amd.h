@@ -171,9 +171,11 @@ int cgfdm_forward_record(cgfdm_solver* s, int nsteps, int checkpoint_every, doub
  * needed, by the next cgfdm_forward_record). */
 int cgfdm_adjoint(cgfdm_solver* s, const double* src, double* gmu, double* glam, double* gb, double* grate);
 
-/* Per-kernel timing with HIP events on the solver stream. enable = 1 starts
- * accumulation (and clears it), 0 stops. out[0..5] = {interior ms, interior
- * launches, surface ms, surface launches, step ms, steps}; out may be NULL.
+/* Per-kernel timing with HIP events on the solver stream, of the launches that are
+ * made without it too. enable = 1 starts accumulation (and clears it), 0 stops.
+ * out[0..5] = {interior ms, interior launches, surface ms, surface launches, step
+ * ms, steps}; a stage in one launch (cg_stage) counts as interior, and the surface's
+ * figures are then zero; out may be NULL.
  * AWENO: {face-flux ms, launches, update ms, launches, step ms, steps}. */
 int cgfdm_timing(cgfdm_solver* s, int enable, double* out);
 
@@ -198,7 +200,9 @@ int cgfdm_grid_ranges_noalloc(int nx, int ny, int nz, const float* coord, const 
 /* Name of the kernel the solver launches (no reference counterpart; for profiles
  * and reports): which = 0 the interior stage kernel (CGFDM: cg_cell, cg_zreg, ...)
  * or the face-flux kernel (AWENO), 1 the surface kernel (CGFDM) or the update
- * kernel (AWENO). NULL for a bad handle or index. */
+ * kernel (AWENO). Small grids take both CGFDM kernels in one, cg_stage, which is then
+ * the answer to both, and both AWENO update kernels in one, aw_update_both. NULL for a
+ * bad handle or index. */
 const char* cgfdm_kernel_name(cgfdm_solver* s, int which);
 
 /* Device bytes held by the solver. */

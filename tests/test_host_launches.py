@@ -81,3 +81,30 @@ assert 1 < pieces(g) < 40 and g.device_bytes() == sim.used <= sim.limit
 copies(g)
 g.close()
 """)
+
+
+@pytest.mark.parametrize("scheme,precision,coef,size", [
+    ("CGFDM", 4, 0, (24, 20, 16)), ("CGFDM", 4, 1, (24, 20, 16)), ("CGFDM", 8, 0, (24, 20, 16)),
+    ("CGFDM", 4, 0, (130, 100, 26)), ("AWENO", 4, 0, (24, 20, 16)), ("AWENO", 8, 0, (24, 20, 16)),
+    ("AWENO", 4, 0, (70, 90, 40))])
+@pytest.mark.parametrize("free_surface", [True, False])
+def test_timing_and_names_describe_the_launches_of_a_step(scheme, precision, coef, size, free_surface):
+    """Kernel timing times the launches that a step makes without it, and the kernel names are names of them."""
+    run(f"""
+m = M.small_config(nx={size[0]}, ny={size[1]}, nz={size[2]}, npml=4, nt=8, free_surface={free_surface})
+g = S.Solver(m, precision={precision}, coef_storage={coef}, scheme=S.SCHEME_{scheme})
+sim.launches.clear()
+g.step(2)
+plain = list(sim.launches)
+sim.launches.clear()
+g.timing(True)
+g.step(2)
+t = g.timing(False)
+assert sim.launches == plain, (plain, sim.launches)
+names = [n for n, _ in plain]
+stages = 4 if '{scheme}' == 'CGFDM' else 3
+assert names.count(g.kernel_name(0)) == 2 * stages == t['interior_n'], (g.kernel_name(0), names)
+if '{scheme}' == 'AWENO' or {free_surface}:
+    assert names.count(g.kernel_name(1)) == 2 * stages, (g.kernel_name(1), names)
+    assert t['surface_n'] == (0 if g.kernel_name(1) == 'cg_stage' else 2 * stages)
+""")
