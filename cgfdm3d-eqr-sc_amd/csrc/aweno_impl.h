@@ -705,9 +705,11 @@ void launch_update(const StageArgs<R>& a, int nx, int ny, hipStream_t st) {
   // the top three layers and the rest write disjoint cells and read only the stage
   // input and the face fluxes
   const dim3 block(256), gtop((nx + 63) / 64, (ny + 3) / 4, 3);
-  if (const long long both = one_update_blocks(a, nx, ny)) {
-    aw_update_both<R><<<dim3((unsigned)both), block, 0, st>>>(a, nx, ny);
-    return;
+  if constexpr (sizeof(R) == 4) {
+    if (const long long both = one_update_blocks(a, nx, ny)) {
+      aw_update_both<R><<<dim3((unsigned)both), block, 0, st>>>(a, nx, ny);
+      return;
+    }
   }
   const long long nb = cg::interior_blocks(a.XE - 2 * H, a.NY, a.NZ, a.rtx, a.rty);
   aw_update_top<R, false><<<gtop, block, 0, st>>>(a, nx, ny);

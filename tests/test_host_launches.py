@@ -108,3 +108,11 @@ if '{scheme}' == 'AWENO' or {free_surface}:
     assert names.count(g.kernel_name(1)) == 2 * stages, (g.kernel_name(1), names)
     assert t['surface_n'] == (0 if g.kernel_name(1) == 'cg_stage' else 2 * stages)
 """)
+
+
+def test_no_fp64_kernel_of_both_updates():
+    """The one launch of both ME-AWENO updates is for FP32 only: an FP64 instance would be compiled for nothing."""
+    lib = os.path.join(os.path.dirname(HERE), "cgfdm3d-eqr-sc_amd", "cgfdm_amd", "libcgfdm_amd.so")
+    with open(lib, "rb") as f:
+        names = f.read()
+    assert b"aw14aw_update_bothIf" in names and b"aw14aw_update_bothId" not in names
