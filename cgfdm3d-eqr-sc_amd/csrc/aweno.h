@@ -42,6 +42,7 @@ inline long long one_update_blocks(const StageArgs<R>& a, int nx, int ny) {
 // first, then x, z and the top layers.
 void launch_march_y(const StageArgs<float>& a, int nx, int ny, hipStream_t st);
 void launch_march_xz(const StageArgs<float>& a, int nx, int ny, hipStream_t st);
+bool march_pays(int nx, int ny, int nz, int rtx, int rty);
 template <class R>
 void launch_char_surface(R* W, const R* cjm, int nx, int ny, int NX, int NZ, long long N, long long S, hipStream_t st);
 template <class R>

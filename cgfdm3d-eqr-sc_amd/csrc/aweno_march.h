@@ -353,7 +353,7 @@ aw_xzstep(StageArgs<float> a, int nbx, int chunk, unsigned nb8) {
 // per SIMD, and a second one on each costs about two thirds of the first's time.
 // Measured in us per stage at 200 x 180 x 100 with chunks of 8, 16, 32 cells: 539,
 // 492, 544; at 128 x 120 x 80: 210, 188, 276.
-inline int march_cells(long long units, int cells) {
+inline int march_cells(long long units, int cells, double* cost_of = nullptr) {
   int best = cells;
   double least = 0.0;
   for (int n = 1; n <= cells; ++n) {
@@ -364,7 +364,31 @@ inline int march_cells(long long units, int cells) {
     least = cost;
     best = c;
   }
+  if (cost_of) *cost_of = least;
   return best;
+}
+
+// Whether the marching kernels are the faster ones: us per step from the costs of
+// their two launches and the blocks of the top layers, against the blocks of the two
+// kernels with the flux array.
+// The figures are fitted to both paths on 170 grids of 0.1 to 12 million cells with
+// extents from 4 to 2000, most of them near the line. On 66 others the path taken is
+// the slower one by more than 6 % once (536 x 77 x 17, 0.487 ms for 0.414), and a mean
+// 0.4 % slower than the better one; a line at a number of cells does worse, since
+// marching gains with the depth and with the lanes that a row fills. ms per step with
+// the array and marching: 59 x 90 x 78 0.320 and 0.397, 400 x 400 x 6 0.655 and 0.786,
+// 900 x 800 x 6 2.78 and 3.13, 166 x 80 x 46 0.392 and 0.387, 512 x 500 x 60 6.37 and
+// 4.18, 320 x 300 x 200 7.72 and 4.83.
+bool march_pays(int nx, int ny, int nz, int rtx, int rty) {
+  const int nk = nz - 3;  // at least 1: a grid has four planes
+  const long long bx = (nx + 63) / 64;
+  double cy, cz;
+  march_cells(bx * nk, ny, &cy);
+  march_cells((long long)x_waves(nx + 2 * H) * ny, nk, &cz);
+  const double march = 33.0 + 10.9 * cy + 11.8 * cz + 0.5 * (double)(bx * ((ny + 3) / 4));
+  const double array = 95.0 + 0.0488 * (double)(cg::interior_blocks(nx, ny + 1, nz + 1, rtx, rty) +
+                                               cg::interior_blocks(nx, ny + 2 * H, nz + 2 * H, rtx, rty));
+  return march < array;
 }
 
 inline unsigned march_blocks8(long long waves) { return (unsigned)(((waves + 3) / 4 + 7) / 8); }

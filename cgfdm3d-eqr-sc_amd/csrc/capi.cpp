@@ -1360,10 +1360,8 @@ struct AwenoSolver : SolverBase {
   // CGFDM_INTERIOR_RTX (0..64) / _RTY (1..64) override it
   int rty = 2;
   int rtx = 0;
-  // FP32: marching kernels without the flux array (aweno_march.h) from 400000
-  // cells on, where they have enough columns to fill the chip: us per stage
-  // 97 against 66 at 64 x 60 x 40, 131 against 156 at 96 x 90 x 60, 1395 against
-  // 2070 at 512 x 500 x 60. CGFDM_AWENO_MARCH (0 or 1) overrides the rule.
+  // FP32: marching kernels without the flux array (aweno_march.h) where they are the
+  // faster ones (march_pays); CGFDM_AWENO_MARCH (0 or 1) overrides the rule
   bool march = false;
 
   int init(const cgfdm_desc& dd, const float* coord, const float* medium) override {
@@ -1426,7 +1424,7 @@ struct AwenoSolver : SolverBase {
     dfree(cjm_t);
     for (int q = 0; q < 3; ++q)
       if ((rc = galloc(&buf[q], 9 * N))) return rc;
-    march = sizeof(R) == 4 && (double)d.nx * d.ny * d.nz >= 400000.0;
+    march = sizeof(R) == 4 && aw::march_pays(d.nx, d.ny, d.nz, rtx, rty);
     if (const char* e = std::getenv("CGFDM_AWENO_MARCH")) march = sizeof(R) == 4 && std::atoi(e) != 0;
     if (!march && (rc = galloc(&F, 27 * N))) return rc;
     if ((rc = dalloc(&pgv, 2LL * d.nx * d.ny))) return rc;

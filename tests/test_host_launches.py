@@ -116,3 +116,15 @@ def test_no_fp64_kernel_of_both_updates():
     with open(lib, "rb") as f:
         names = f.read()
     assert b"aw14aw_update_bothIf" in names and b"aw14aw_update_bothId" not in names
+
+
+@pytest.mark.parametrize("size,march", [((59, 90, 78), False), ((400, 400, 6), False), ((64, 60, 40), False),
+                                        ((250, 240, 4), False), ((100, 150, 130), True), ((160, 150, 90), True)])
+def test_marching_kernels_where_they_are_faster(size, march):
+    """ME-AWENO in FP32: grids that are thin, or narrow with half-empty waves, take the kernels with the flux array,
+    which are the faster ones there by a fifth (measured); deep ones of a million cells and more march."""
+    run(f"""
+m = M.small_config(nx={size[0]}, ny={size[1]}, nz={size[2]}, npml=0, nt=4, hills=0, layered=False)
+g = S.Solver(m, precision=4, scheme=S.SCHEME_AWENO)
+assert g.kernel_name(0) == ('aw_yflux' if {march} else 'aw_faces'), g.kernel_name(0)
+""")
