@@ -695,8 +695,10 @@ __global__ void aw_record(const R* __restrict__ W, const R* __restrict__ cjm, lo
 template <class R>
 void launch_faces(const StageArgs<R>& a, hipStream_t st) {
   const long long nb = cg::interior_blocks(a.XE - 2 * H, a.NY - 5, a.NZ - 5, a.rtx, a.rty);
-  // a few blocks, all resident at once: the three directions side by side instead of
-  // one after another in each thread (48 x 44 x 20: 158 -> 142 us per step)
+  // few blocks: the three directions side by side instead of one after another in
+  // each thread. us per step without and with: 48 x 44 x 20 99 and 85, 64 x 70 x 44
+  // (about 1000 blocks) 190 and 174; 128 x 60 x 40, above the line, still 223 and 218.
+  // FP64 170 and 154, 288 and 271, 356 and 346.
   aw_faces<R><<<dim3((unsigned)nb, nb <= 1024 ? 3 : 1), dim3(256), 0, st>>>(a);
 }
 

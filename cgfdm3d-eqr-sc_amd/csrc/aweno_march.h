@@ -372,7 +372,7 @@ inline int march_cells(long long units, int cells, double* cost_of = nullptr) {
 // their two launches and the blocks of the top layers, against the blocks of the two
 // kernels with the flux array.
 // The figures are fitted to both paths on 170 grids of 0.1 to 12 million cells with
-// extents from 4 to 2000, most of them near the line. On 66 others the path taken is
+// extents from 4 to 2000, most of them near the line. On 68 others the path taken is
 // the slower one by more than 6 % once (536 x 77 x 17, 0.487 ms for 0.414), and a mean
 // 0.4 % slower than the better one; a line at a number of cells does worse, since
 // marching gains with the depth and with the lanes that a row fills. ms per step with

@@ -156,8 +156,8 @@ __device__ __forceinline__ void pml_face(const FaceBuf<R>& F, long long pos, con
 // global memory) and the z-marching ones (from an LDS plane or registers). All of
 // an axis' loads are issued before its arithmetic.
 // ---------------------------------------------------------------------------
-// Streaming accesses of a stage (coefficients, RK base and accumulator, the
-// two outputs) are used once per cell: they carry the non-temporal hint so
+// Streaming accesses of a stage (coefficients, RK base and earlier stage states,
+// the output) are used once per cell: they carry the non-temporal hint so
 // that they do not displace the stencil rows of W in L2 (measured on the
 // 512x512x256 workload: interior kernel 5.20 -> 5.06 ms per launch).
 template <class T>
@@ -977,9 +977,9 @@ __global__ __launch_bounds__(256) void cg_surface(StageArgs<R> a, const TM* __re
   surface_block<R, TM, FB1, FB2, FB3, STAGE>(a, coef, s, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// Both in one launch, the surface blocks first, for grids whose blocks are all
-// resident at once (launch_stage): there the two kernels are bound by the latency
-// of their loads, one after the other, and registers for more waves have no use.
+// Both in one launch, the surface blocks first, for grids of one or two rounds of
+// blocks (one_launch_blocks): there the two kernels are bound by the latency of their
+// loads, one after the other, and registers for more waves have little use.
 template <class R, class TM, int FB1, int FB2, int FB3, int STAGE>
 __global__ __launch_bounds__(256) void cg_stage(StageArgs<R> a, const TM* __restrict__ coef, SurfArgs<R> s) {
   const int ntx = (a.nx + 63) / 64, nty = (a.ny + 3) / 4, b = blockIdx.x, n = 3 * ntx * nty;
