@@ -103,8 +103,8 @@ __device__ __forceinline__ void weno5_pair(double wm2, double wm1, double w0, do
   up = weno5_side(fma(3.0 * f1, f1, Tm1), fma(3.0 * C0, C0, T0), fma(3.0 * f3, f3, T1), PB, 2.0 * PA, Pp);
 }
 
-// One side with the weights as they are defined, for faces whose values from
-// weno5_pair are not finite.
+// One side with the weights as they are defined, for faces whose flux from
+// weno5_pair is not finite (face_flux).
 __device__ __forceinline__ double weno5_wide(double u1, double u2, double u3, double u4, double u5) {
   constexpr double eps = 12e-6 / (3.0 * 0.3333333333);
   const double a1 = u3 - 2.0 * u4 + u5, e1 = 3.0 * u3 - 4.0 * u4 + u5;
@@ -144,8 +144,8 @@ __device__ __forceinline__ R pl(const R* base, long long N, int c, unsigned o) {
 
 // Lax-Friedrichs face flux of direction d at face q+1/2
 // (wave_deriv_alternative_flux_FD_{x,y,z}); o is the byte offset of cell q,
-// sb the byte stride of direction d.
-template <class R>
+// sb the byte stride of direction d. WIDE (FP64): from weno5_wide.
+template <class R, bool WIDE = false>
 __device__ __forceinline__ void face_values(const StageArgs<R>& a, unsigned o, unsigned sb, int d, R (&F)[9]) {
   const long long N = a.N;
   const R n1 = pl(a.cjm, N, 3 * d + 0, o), n2 = pl(a.cjm, N, 3 * d + 1, o), n3 = pl(a.cjm, N, 3 * d + 2, o);
@@ -156,7 +156,14 @@ __device__ __forceinline__ void face_values(const StageArgs<R>& a, unsigned o, u
     const R* w = a.win + v * N;
     const R wm2 = *at(w, o - 2 * sb), wm1 = *at(w, o - sb), w0 = *at(w, o), wp1 = *at(w, o + sb),
             wp2 = *at(w, o + 2 * sb), wp3 = *at(w, o + 3 * sb);
-    weno5_pair(wm2, wm1, w0, wp1, wp2, wp3, um[v], up[v]);
+    if constexpr (WIDE) {
+      um[v] = weno5_wide(wm2, wm1, w0, wp1, wp2);
+      __builtin_amdgcn_sched_barrier(0);  // one side after the other: all at once would take 256 registers
+      up[v] = weno5_wide(wp3, wp2, wp1, w0, wm1);
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      weno5_pair(wm2, wm1, w0, wp1, wp2, wp3, um[v], up[v]);
+    }
   }
   if constexpr (sizeof(R) == 4) {
     // the flux is linear in the state: F(u+) + F(u-) = F(u+ + u-), one flux
@@ -168,34 +175,11 @@ __device__ __forceinline__ void face_values(const StageArgs<R>& a, unsigned o, u
 #pragma unroll
     for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (F[v] - a.alpha * (up[v] - um[v]));
   } else {
-    auto flux = [&](R n1, R n2, R n3, R mu, R lam, R b) {
-      R fm[9], fp[9];
-      phys_flux<R>(um, n1, n2, n3, mu, lam, b, fm);
-      phys_flux<R>(up, n1, n2, n3, mu, lam, b, fp);
+    R fm[9], fp[9];
+    phys_flux<R>(um, n1, n2, n3, mu, lam, b, fm);
+    phys_flux<R>(up, n1, n2, n3, mu, lam, b, fp);
 #pragma unroll
-      for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (fp[v] + fm[v] - a.alpha * (up[v] - um[v]));
-    };
-    flux(n1, n2, n3, mu, lam, b);
-    // an overflow in weno5_side makes one of its three weights infinite, so its
-    // numerator infinite or NaN, and its value and the flux not finite: one test per
-    // face (a step at 150 x 140 x 90 takes 2.056 ms without it and 2.058 with it)
-    R s = R(0);
-#pragma unroll
-    for (int v = 0; v < 9; ++v) s += F[v];
-    if (!(fabs(s) < __builtin_huge_val())) {
-      unsigned q = o;
-      asm("" : "+v"(q));  // loaded again: kept from above the nine fields would take 108 registers
-#pragma unroll
-      for (int v = 0; v < 9; ++v) {
-        auto w = [&](unsigned off) { return *at(a.win + v * N, off); };
-        um[v] = weno5_wide(w(q - 2 * sb), w(q - sb), w(q), w(q + sb), w(q + 2 * sb));
-        __builtin_amdgcn_sched_barrier(0);  // one side after the other: all at once would take 256 registers
-        up[v] = weno5_wide(w(q + 3 * sb), w(q + 2 * sb), w(q + sb), w(q), w(q - sb));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      flux(pl(a.cjm, N, 3 * d + 0, q), pl(a.cjm, N, 3 * d + 1, q), pl(a.cjm, N, 3 * d + 2, q), pl(a.cjm, N, C_MU, q),
-           pl(a.cjm, N, C_LAM, q), pl(a.cjm, N, C_B, q));
-    }
+    for (int v = 0; v < 9; ++v) F[v] = R(0.5) * (fp[v] + fm[v] - a.alpha * (up[v] - um[v]));
   }
 }
 
@@ -211,6 +195,22 @@ __device__ __forceinline__ void face_flux(const StageArgs<R>& a, unsigned o, uns
   for (int v = 0; v < 9; ++v) {
     if constexpr (sizeof(R) == 4) __builtin_nontemporal_store(f[v], at(F + v * a.N, o));
     else *at(F + v * a.N, o) = f[v];
+  }
+  if constexpr (sizeof(R) == 8) {
+    // an overflow in weno5_side makes one of its three weights infinite, so its
+    // numerator infinite or NaN, and its value and the flux not finite: one test per
+    // face, after the stores, where it adds no register to them. us per step without
+    // it and with it: 150 x 140 x 90 2058 and 2056, 96 x 64 x 49 366 and 367,
+    // 36 x 51 x 20 166 and 171.
+    R s = f[0];
+#pragma unroll
+    for (int v = 1; v < 9; ++v) s += f[v];
+    if (!(fabs(s) < __builtin_huge_val())) {
+      asm("" : "+v"(o));  // loaded again: kept from above the nine fields would take 108 registers
+      face_values<R, true>(a, o, sb, d, f);
+#pragma unroll
+      for (int v = 0; v < 9; ++v) *at(F + v * a.N, o) = f[v];
+    }
   }
 }
 
@@ -235,7 +235,11 @@ __global__ void __launch_bounds__(256) aw_faces(StageArgs<R> a) {
   const int only = gridDim.y == 3 ? (int)blockIdx.y : -1;
   if (ji && ki && only <= 0) {
     face_flux<R>(a, o, (unsigned)sizeof(R), 0);
-    if (i == H) face_flux<R>(a, o - (unsigned)sizeof(R), (unsigned)sizeof(R), 0);
+    if (i == H) {
+      unsigned q = o - (unsigned)sizeof(R);
+      if constexpr (sizeof(R) == 8) asm("" : "+v"(q));  // nothing is kept for this face from the one above
+      face_flux<R>(a, q, (unsigned)sizeof(R), 0);
+    }
   }
   if (ki && (only < 0 || only == 1)) face_flux<R>(a, o, a.rowb, 1);
   if (ji && (only < 0 || only == 2)) face_flux<R>(a, o, a.planeb, 2);
